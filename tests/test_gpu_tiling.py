@@ -178,3 +178,51 @@ def test_plan_from_csr_matches_host_tiles(gpu, config, prec):
     finally:
         host_plan.close()
         dev_plan.close()
+
+
+# A row-block's entries are sorted by a wave (up to 1024, in registers of 1,
+# 2, 4, 8 or 16 entries per lane), a workgroup (up to 8192) or globally: the
+# edges of each, in blocks beside small and empty ones, with duplicates (some
+# in one slot, in runs longer than a 64-entry step) and unsorted rows.
+@pytest.mark.parametrize("entries", [1, 63, 64, 65, 128, 129, 256, 257, 512, 513, 1023, 1024, 1025, 2048, 2049, 4096,
+                                     4097, 8191, 8192, 8193, 20001])
+@pytest.mark.parametrize("prec,bm", [(0, 8), (1, 16), (1, 64)])
+def test_device_tiles_block_sizes(gpu, orc, entries, prec, bm):
+    rng = np.random.default_rng(entries)
+    rows, cols = 3 * bm + 5, 30011
+    # block 0 empty, block 1 with `entries`, block 2 with a few, a ragged one
+    length = np.zeros(rows, np.int64)
+    part = rng.multinomial(entries, rng.dirichlet(np.ones(bm) * 0.5))
+    length[bm:2 * bm] = part
+    length[2 * bm:] = rng.integers(0, 7, rows - 2 * bm)
+    rp = np.concatenate([[0], np.cumsum(length)]).astype(np.int32)
+    ci = rng.integers(0, cols, rp[-1]).astype(np.int32)
+    same = rng.random(len(ci)) < 0.3
+    ci[same] = ci[0] if len(ci) else 0              # one column many times
+    store, bits = values_for(rng, len(ci), prec)
+    check_vs_oracle(gpu, orc, rows, cols, rp, ci, prec, bm, store, bits, f"{entries} entries in a block")
+
+
+def test_device_tiles_many_columns(gpu, orc):
+    # more than 2^22 columns: 64-bit sort keys in the wave sort
+    rng = np.random.default_rng(11)
+    rows, cols = 101, (1 << 22) + 9
+    rp, ci = random_csr(rng, rows, cols, 90, dup=True, empty_frac=0.1)
+    ci[:4] = [cols - 1, 0, cols - 1, 1 << 22][:min(4, len(ci))]
+    for prec in (0, 1):
+        store, bits = values_for(rng, len(ci), prec)
+        check_vs_oracle(gpu, orc, rows, cols, rp, ci, prec, 8, store, bits, "many columns")
+
+
+@pytest.mark.parametrize("bm,bn", [(8, 1), (8, 5), (16, 32), (64, 7), (64, 32)])
+@pytest.mark.parametrize("prec", [0, 1])
+def test_device_tiles_other_widths(gpu, orc, prec, bm, bn):
+    # tile widths other than the classes' own go through the generic kernel
+    rng = np.random.default_rng(100 * bm + bn)
+    rows, cols = 300, 700
+    rp, ci = random_csr(rng, rows, cols, 60, dup=True, empty_frac=0.2)
+    store, bits = values_for(rng, len(ci), prec)
+    sub = gpu.Csr(rows, cols, rp, ci, store, prec)
+    say(f"device tiles {bm}x{bn} prec={prec}")
+    d = gpu.tile_create_device(sub, cols, bm, prec, bn)
+    assert_same(d, orc.tile_create(rows, cols, rp, ci, bits, prec, bm, bn), prec, f"{bm}x{bn}")

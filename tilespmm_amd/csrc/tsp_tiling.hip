@@ -2,31 +2,37 @@
 // src/csr2tile.h:15-379,724-795 moved onto MI355X), bit-exact with the host
 // conversion (tilespmm_amd/host/tiles.cpp).
 //
-//   1. key[e] = (row-block of entry e, column), value = e; one stable LSD
-//      radix sort (rocPRIM) of all pairs.  Entries of one (block, column)
-//      pair become a contiguous run that keeps the CSR order.
-//   2. run heads -> exclusive scan -> run ids.  A block's runs are its sorted
-//      distinct columns; the rank of a run inside its block is its run id
-//      minus the run id at the block's first entry, and the block's distinct
-//      count d is the difference at its ends (the sort keeps blocks in place,
-//      so block b's entries still start at ptr[b*BM]).
-//   3. ceil(d/BN) tiles per block, exclusive scan -> tile_ptr; tile_colidx is
-//      the distinct list cut into BN-wide tiles, padded with the last column.
-//   4. one thread per run walks its entries in CSR order: slot
-//      (local row, rank % BN) of tile rank / BN, per-tile entry count, bitmap
-//      bit, and a sequential add into the canonical row-major slot with the
-//      value type's rounding after every add (fp16: fp32 add then round to
-//      half).  A slot belongs to exactly one run, so duplicates accumulate in
-//      CSR order exactly as on the host.
-//   5. exclusive scan of the per-tile counts -> tile_nnz.
-// Work is O(nnz) with no per-row serial loop, so hub rows of power-law
-// matrices cost no more than their entries.
+//   1. Each row-block's entries are sorted by (column, position) where they
+//      lie: a block of up to kSmall entries by one wave in registers, up to
+//      kMedium by one workgroup through LDS, larger ones (a dense row of a
+//      circuit, the hubs of a power-law graph) by one rocPRIM radix sort over
+//      the entries of all such blocks.  The only scratch is one word per
+//      entry: its position inside the block, bit 31 set where a new column
+//      starts.  Entries of one (block, column) pair keep the CSR order.
+//   2. ceil(distinct / BN) tiles per block; one chained scan -> tile_ptr.
+//   3. One wave per block (per kSmall sorted entries of a larger block) walks
+//      its sorted entries, builds its tiles a few at a time in LDS -- values,
+//      occupancy bits -- and writes them with whole lines, zeros included, so
+//      no array is cleared first.  An entry's slot is (its local row, its
+//      column's rank % BN) of tile rank / BN; the ranks are prefix counts of
+//      the bit-31 flags.  A slot's first entry adds up its duplicates in CSR
+//      order with the value type's rounding after every add (fp16: fp32 add
+//      then round to half), exactly as on the host.  A tile's first sorted
+//      entry is tile_nnz, its columns tile_colidx.
+//
+// The conversion is bound by memory traffic: it reads the column indices
+// twice, the values once, the 4-byte scratch twice, and writes the tiles
+// once.  RMAT scale 22 (128M entries) to tf32 8-row tiles: 8.9 ms of kernels,
+// against 28 ms for a global radix sort of 8-byte keys over all entries with
+// cleared output arrays filled by one thread per column run.
 #include <cstring>
 #include <hip/hip_runtime.h>
 #include <rocprim/rocprim.hpp>
+#include <limits.h>
 #include <stdint.h>
 
 #include <mutex>
+#include <type_traits>
 
 #include "../../include/tilespmm_hip.h"
 #include "tsp_kernels.h"
@@ -55,80 +61,416 @@ int bits_for(long long v)     // bits to hold values 0 .. v-1
     return b;
 }
 
-// bptr[b] = ptr[min(rows, b*BM)], b = 0..tilem
-__global__ void block_ptr_kernel(const int *__restrict__ ptr, int rows, int tilem, int bm, int *__restrict__ bptr)
+// ---- 1. the sorted entries of every row-block -------------------------------
+constexpr int kSmallBits = 10;
+constexpr int kSmall = 1 << kSmallBits;    // entries one wave sorts, and walks in step 3
+constexpr int kMedium = 8192;              // entries one workgroup sorts (64 KB of LDS)
+constexpr int kMediumThreads = 1024;
+constexpr unsigned kHead = 0x80000000u;    // sorted entry that starts a new column
+
+// kSmall sorted entries of a block with more than that: positions p0 ..,
+// rank0 columns start before them, rank1 before the next unit.
+struct Unit {
+    int b, p0, rank0, rank1;
+};
+// A block with more than kSmall entries, its first unit and (global sort)
+// its first entry there.
+struct Big {
+    int b, unit0;
+    long long off;
+};
+// Zeroed before each conversion.
+struct Counters {
+    unsigned long long huge;               // (blocks << 40) + entries of the globally sorted blocks
+    long long total;                       // tiles
+    int bad;                               // a column outside [0, colA), or row pointers out of order
+    int nunits, nmedium;
+    int ticket;                            // of the chained scan
+};
+
+// The CSR entries of row-block b.  (Entries outside ptr[0] .. ptr[rows]
+// belong to the first and the last row.)
+__device__ __forceinline__ void block_range(const int *__restrict__ ptr, int rows, int nnz, int bm, int tilem, int b,
+                                            int &s, int &n)
 {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b > tilem) return;
     const long long r = (long long)b * bm;
-    bptr[b] = ptr[r < rows ? r : rows];
+    s = b == 0 ? 0 : min(max(ptr[r], 0), nnz);
+    const int e = b == tilem - 1 ? nnz : min(max(ptr[r + bm], 0), nnz);
+    n = max(e - s, 0);
+    (void)rows;
 }
 
-// one thread per entry: key = (block << cbits) | col, value = entry index,
-// lrow = row inside the block.  The row comes from a binary search of ptr.
-__global__ void key_kernel(const int *__restrict__ ptr, const int *__restrict__ idx, int rows, long long nnz,
-                           int bm, int cbits, int colA, unsigned long long *__restrict__ key,
-                           int *__restrict__ ent, uint8_t *__restrict__ lrow, int *__restrict__ bad)
+template <typename K>
+__device__ __forceinline__ void order(K &a, K &b)
 {
-    const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= nnz) return;
-    int lo = 0, hi = rows - 1;                 // last row r with ptr[r] <= e
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (ptr[mid] <= e) lo = mid;
-        else hi = mid - 1;
-    }
-    const int c = idx[e];
-    if (c < 0 || c >= colA) atomicAdd(bad, 1);
-    const unsigned cc = (unsigned)c & ((1u << cbits) - 1u);
-    key[e] = ((unsigned long long)(lo / bm) << cbits) | cc;
-    ent[e] = (int)e;
-    lrow[e] = (uint8_t)(lo % bm);
+    const K lo = a < b ? a : b, hi = a < b ? b : a;
+    a = lo;
+    b = hi;
 }
 
-__global__ void head_kernel(const unsigned long long *__restrict__ key, long long n, int *__restrict__ flag)
+// One stage of a bitonic merge over elements thread * R + r: element i meets
+// element i ^ j, or i ^ (2j - 1) in the first stage of a merge (FLIP, which
+// keeps every run ascending).  `other(v, d)` gives thread t the value that
+// thread t ^ d passes.
+template <int J, bool FLIP, int R, typename K, typename F>
+__device__ __forceinline__ void merge_stage(K (&x)[R], int t, F &&other)
 {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    flag[i] = (i == 0 || key[i] != key[i - 1]) ? 1 : 0;
-}
-
-// run r starts at sorted position i; its column goes to dcols[r]
-__global__ void run_scatter_kernel(const unsigned long long *__restrict__ key, const int *__restrict__ flag,
-                                   const int *__restrict__ run, long long n, unsigned cmask,
-                                   int *__restrict__ run_start, int *__restrict__ dcols)
-{
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    if (flag[i]) {
-        run_start[run[i]] = (int)i;
-        dcols[run[i]] = (int)(key[i] & cmask);
+    if constexpr (J < R) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int p = FLIP ? r ^ (2 * J - 1) : r ^ J;
+            if (p > r) order(x[r], x[p]);
+        }
+    } else {
+        constexpr int D = FLIP ? 2 * J / R - 1 : J / R;
+        const bool upper = (t & (J / R)) != 0;
+        K y[R];
+        other(x, y, D, FLIP);
+#pragma unroll
+        for (int r = 0; r < R; ++r) x[r] = (y[r] < x[r]) == !upper ? y[r] : x[r];
     }
 }
 
-// per block: first run id and distinct count; tiles ceil(d/BN)
-__global__ void block_runs_kernel(const int *__restrict__ bptr, const int *__restrict__ run, int tilem, int bn,
-                                  int *__restrict__ dstart, int *__restrict__ nt)
+template <int J, int R, typename K, typename F>
+__device__ __forceinline__ void merge_rest(K (&x)[R], int t, F &&other)
 {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
+    if constexpr (J >= 1) {
+        merge_stage<J, false>(x, t, other);
+        merge_rest<J / 2>(x, t, other);
+    }
+}
+
+// Sorts N elements, ascending, held as element thread * R + r.
+template <int K2, int N, int R, typename K, typename F>
+__device__ __forceinline__ void bitonic(K (&x)[R], int t, F &&other)
+{
+    if constexpr (K2 <= N) {
+        merge_stage<K2 / 2, true>(x, t, other);
+        merge_rest<K2 / 4>(x, t, other);
+        bitonic<K2 * 2, N>(x, t, other);
+    }
+}
+
+// Sorts the n <= 64 R entries of a block at CSR position s, one wave; writes
+// their sorted words and returns the number of distinct columns.
+template <typename K, int R>
+__device__ __forceinline__ int sort_small(const int *__restrict__ idx, int s, int n, unsigned cmask, int colA, int lane,
+                                          unsigned *__restrict__ words, bool &bad)
+{
+    K x[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int i = r * 64 + lane;
+        x[r] = ~(K)0;                      // past every entry
+        if (i < n) {
+            const unsigned c = (unsigned)idx[s + i];
+            bad |= c >= (unsigned)colA;
+            x[r] = (K)(c & cmask) << kSmallBits | (unsigned)i;
+        }
+    }
+    bitonic<2, 64 * R>(x, lane, [](const K (&v)[R], K (&y)[R], int d, bool flip) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) y[r] = __shfl_xor(v[flip ? R - 1 - r : r], d);
+    });
+    K before = __shfl_up(x[R - 1], 1);
+    int distinct = 0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int i = lane * R + r;
+        const bool head = i < n && (i == 0 || (x[r] >> kSmallBits) != (before >> kSmallBits));
+        before = x[r];
+        distinct += __popcll(__ballot(head));
+        if (i < n) words[s + i] = ((unsigned)x[r] & (kSmall - 1)) | (head ? kHead : 0u);
+    }
+    return distinct;
+}
+
+// One wave per row-block.  K: the type of a sort key, column << kSmallBits |
+// position (32 bits for up to 2^22 columns).
+template <typename K>
+__global__ __launch_bounds__(kThreads) void sort_blocks_kernel(const int *__restrict__ ptr, const int *__restrict__ idx,
+                                                               int rows, int nnz, int bm, int bn, int tilem,
+                                                               unsigned cmask, int colA, unsigned *__restrict__ words,
+                                                               int *__restrict__ nt, Big *__restrict__ medium,
+                                                               int medium_cap, Big *__restrict__ huge, int huge_cap,
+                                                               int unit_cap, Counters *__restrict__ cnt)
+{
+    const int b = (int)((blockIdx.x * (long long)kThreads + threadIdx.x) >> 6), lane = threadIdx.x & 63;
     if (b >= tilem) return;
-    const int s = run[bptr[b]], e = run[bptr[b + 1]];
-    dstart[b] = s;
-    nt[b] = (e - s + bn - 1) / bn;
+    int s, n;
+    block_range(ptr, rows, nnz, bm, tilem, b, s, n);
+    s = __builtin_amdgcn_readfirstlane(s);
+    n = __builtin_amdgcn_readfirstlane(n);
+    bool bad = false;
+    int d = 0;
+    if (n > kSmall) {
+        if (lane == 0) {
+            const int ns = (n + kSmall - 1) / kSmall;
+            const int u = atomicAdd(&cnt->nunits, ns);
+            bad = u < 0 || u > unit_cap - ns;    // only row pointers out of order get there
+            if (!bad && n <= kMedium) {
+                const int j = atomicAdd(&cnt->nmedium, 1);
+                bad = j < 0 || j >= medium_cap;
+                if (!bad) medium[j] = Big{b, u, 0};
+            } else if (!bad) {
+                const unsigned long long at = atomicAdd(&cnt->huge, (1ull << 40) + (unsigned long long)n);
+                const long long j = (long long)(at >> 40);
+                const long long off = (long long)(at & ((1ull << 40) - 1));
+                bad = j >= huge_cap || off + n > nnz;
+                if (!bad) huge[j] = Big{b, u, off};
+            }
+        }
+    } else if (n > 512) {
+        d = sort_small<K, 16>(idx, s, n, cmask, colA, lane, words, bad);
+    } else if (n > 256) {
+        d = sort_small<K, 8>(idx, s, n, cmask, colA, lane, words, bad);
+    } else if (n > 128) {
+        d = sort_small<K, 4>(idx, s, n, cmask, colA, lane, words, bad);
+    } else if (n > 64) {
+        d = sort_small<K, 2>(idx, s, n, cmask, colA, lane, words, bad);
+    } else if (n > 0) {
+        d = sort_small<K, 1>(idx, s, n, cmask, colA, lane, words, bad);
+    }
+    if (lane == 0) nt[b] = (d + bn - 1) / bn;
+    if (bad) cnt->bad = 1;
 }
 
-// one work-group per row-block writes its padded column indices
-__global__ void colidx_kernel(const int *__restrict__ tile_ptr, const int *__restrict__ dstart,
-                              const int *__restrict__ dcols, int bn, int *__restrict__ colidx)
+// Sorts one block of at most kMediumThreads * R entries by the workgroup.
+template <int R>
+__device__ __forceinline__ void sort_medium(const int *__restrict__ idx, int s, int n, unsigned cmask, int colA, Big m,
+                                            int bn, unsigned *__restrict__ words, int *__restrict__ nt,
+                                            Unit *__restrict__ units, unsigned long long *lds, int *heads, bool &bad)
 {
-    const int b = blockIdx.x;
-    const int t0 = tile_ptr[b], nt = tile_ptr[b + 1] - t0;
-    if (nt == 0) return;
-    const int s = dstart[b], d = dstart[b + 1] - s;
-    for (int k = threadIdx.x; k < nt * bn; k += blockDim.x)
-        colidx[(size_t)t0 * bn + k] = dcols[s + (k < d ? k : d - 1)];
+    typedef unsigned long long K;
+    const int t = threadIdx.x;
+    K x[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int i = r * kMediumThreads + t;
+        x[r] = ~0ull;
+        if (i < n) {
+            const unsigned c = (unsigned)idx[s + i];
+            bad |= c >= (unsigned)colA;
+            x[r] = (K)(c & cmask) << 32 | (unsigned)i;
+        }
+    }
+    bitonic<2, kMediumThreads * R>(x, t, [&](const K (&v)[R], K (&y)[R], int d, bool flip) {
+        if (d < 64) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) y[r] = __shfl_xor(v[flip ? R - 1 - r : r], d);
+        } else {
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < R; ++r) lds[r * kMediumThreads + t] = v[r];
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < R; ++r) y[r] = lds[(flip ? R - 1 - r : r) * kMediumThreads + (t ^ d)];
+        }
+    });
+    __syncthreads();
+    lds[t] = x[R - 1];
+    __syncthreads();
+    K before = t > 0 ? lds[t - 1] : 0ull;
+    int mine = 0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int i = t * R + r;
+        const bool head = i < n && (i == 0 || (x[r] >> 32) != (before >> 32));
+        before = x[r];
+        mine += __popcll(__ballot(head));
+        if (i < n) words[s + i] = (unsigned)x[r] | (head ? kHead : 0u);
+    }
+    // a wave holds 64 R sorted entries: kSmall / (64 R) waves a unit
+    if ((t & 63) == 0) heads[t >> 6] = mine;
+    __syncthreads();
+    if (t == 0) {
+        constexpr int PW = kSmall / (64 * R);
+        int run = 0;
+        for (int u = 0; u * kSmall < n; ++u) {
+            int k = 0;
+            for (int w = 0; w < PW; ++w) k += heads[u * PW + w];
+            units[m.unit0 + u] = Unit{m.b, u * kSmall, run, run + k};
+            run += k;
+        }
+        nt[m.b] = (run + bn - 1) / bn;
+    }
+    __syncthreads();
 }
 
+// Workgroups share out the medium blocks.
+__global__ __launch_bounds__(kMediumThreads) void sort_medium_kernel(const int *__restrict__ ptr,
+                                                                     const int *__restrict__ idx, int rows, int nnz,
+                                                                     int bm, int bn, int tilem, unsigned cmask,
+                                                                     int colA, unsigned *__restrict__ words,
+                                                                     int *__restrict__ nt,
+                                                                     const Big *__restrict__ medium, int medium_cap,
+                                                                     Unit *__restrict__ units,
+                                                                     Counters *__restrict__ cnt)
+{
+    __shared__ unsigned long long lds[kMedium];
+    __shared__ int heads[kMediumThreads / 64];
+    const int nm = min(cnt->nmedium, medium_cap);
+    bool bad = false;
+    for (int j = blockIdx.x; j < nm; j += gridDim.x) {
+        const Big m = medium[j];
+        int s, n;
+        block_range(ptr, rows, nnz, bm, tilem, m.b, s, n);
+        if (n > 4 * kMediumThreads)
+            sort_medium<8>(idx, s, n, cmask, colA, m, bn, words, nt, units, lds, heads, bad);
+        else if (n > 2 * kMediumThreads)
+            sort_medium<4>(idx, s, n, cmask, colA, m, bn, words, nt, units, lds, heads, bad);
+        else
+            sort_medium<2>(idx, s, n, cmask, colA, m, bn, words, nt, units, lds, heads, bad);
+    }
+    if (bad) cnt->bad = 1;
+}
+
+// Huge blocks: grid (blocks, kHugeY) of workgroups.
+constexpr int kHugeY = 64;
+__global__ __launch_bounds__(kThreads) void huge_keys_kernel(const int *__restrict__ ptr, const int *__restrict__ idx,
+                                                             int rows, int nnz, int bm, int tilem, int cbits, int colA,
+                                                             const Big *__restrict__ huge,
+                                                             unsigned long long *__restrict__ key,
+                                                             unsigned *__restrict__ pos, Counters *__restrict__ cnt)
+{
+    const int j = blockIdx.x;
+    const Big h = huge[j];
+    int s, n;
+    block_range(ptr, rows, nnz, bm, tilem, h.b, s, n);
+    bool bad = false;
+    for (long long i = blockIdx.y * kThreads + threadIdx.x; i < n; i += kHugeY * kThreads) {
+        const unsigned c = (unsigned)idx[s + i];
+        bad |= c >= (unsigned)colA;
+        key[h.off + i] = (unsigned long long)j << cbits | (c & ((1ull << cbits) - 1ull));
+        pos[h.off + i] = (unsigned)i;
+    }
+    if (bad) cnt->bad = 1;
+}
+
+// The sorted words of the huge blocks, and the columns each unit starts
+// (rank1; the ranks follow).
+__global__ __launch_bounds__(kThreads) void huge_words_kernel(const int *__restrict__ ptr, int rows, int nnz, int bm,
+                                                              int tilem, const Big *__restrict__ huge,
+                                                              const unsigned long long *__restrict__ key,
+                                                              const unsigned *__restrict__ pos,
+                                                              unsigned *__restrict__ words, Unit *__restrict__ units)
+{
+    const Big h = huge[blockIdx.x];
+    const int lane = threadIdx.x & 63, wave = blockIdx.y * (kThreads / 64) + (threadIdx.x >> 6);
+    int s, n;
+    block_range(ptr, rows, nnz, bm, tilem, h.b, s, n);
+    for (long long u = wave; u * kSmall < n; u += kHugeY * (kThreads / 64)) {
+        int k = 0;
+        for (int i = 0; i < kSmall; i += 64) {
+            const long long p = u * kSmall + i + lane;
+            const bool in = p < n;
+            const bool head = in && (p == 0 || key[h.off + p] != key[h.off + p - 1]);
+            if (in) words[s + p] = pos[h.off + p] | (head ? kHead : 0u);
+            k += __popcll(__ballot(head));
+        }
+        if (lane == 0) units[h.unit0 + u] = Unit{h.b, (int)(u * kSmall), 0, k};
+    }
+}
+
+// One workgroup per huge block: ranks of its units, its tiles.
+__global__ __launch_bounds__(kThreads) void huge_ranks_kernel(const int *__restrict__ ptr, int rows, int nnz, int bm,
+                                                              int bn, int tilem, const Big *__restrict__ huge,
+                                                              Unit *__restrict__ units, int *__restrict__ nt)
+{
+    using BS = rocprim::block_scan<int, kThreads>;
+    __shared__ typename BS::storage_type st;
+    const Big h = huge[blockIdx.x];
+    int s, n;
+    block_range(ptr, rows, nnz, bm, tilem, h.b, s, n);
+    const int nu = (int)(((long long)n + kSmall - 1) / kSmall);
+    int carry = 0;
+    for (int base = 0; base < nu; base += kThreads) {
+        const int u = base + (int)threadIdx.x;
+        const int v = u < nu ? units[h.unit0 + u].rank1 : 0;
+        int ex = 0, agg = 0;
+        BS().exclusive_scan(v, ex, 0, agg, st, rocprim::plus<int>());
+        if (u < nu) {
+            units[h.unit0 + u].rank0 = carry + ex;
+            units[h.unit0 + u].rank1 = carry + ex + v;
+        }
+        carry += agg;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) nt[h.b] = (carry + bn - 1) / bn;
+}
+
+// ---- 2. chained scan --------------------------------------------------------
+// out[i] = in(0) + .. + in(i - 1) for i = 0 .. n, and the 64-bit total, in
+// one launch: workgroups take tickets in order, publish the sum of their
+// kScanBlock inputs and add up the sums published before theirs (Merrill and
+// Garland's decoupled look-back).  A workgroup only waits for lower tickets,
+// which run already and publish before they wait.  state: 0 = nothing yet,
+// else value << 2 | 1 (the workgroup's own sum) or | 2 (the sum so far);
+// state and ticket are zero at the start.
+constexpr int kScanPer = 8;
+constexpr int kScanBlock = kThreads * kScanPer;
+
+template <typename F>
+__global__ __launch_bounds__(kThreads) void scan_kernel(F in, int n, int *__restrict__ out,
+                                                        unsigned long long *__restrict__ state,
+                                                        int *__restrict__ ticket, long long *__restrict__ total)
+{
+    using BS = rocprim::block_scan<long long, kThreads>;
+    __shared__ typename BS::storage_type st;
+    __shared__ long long before;
+    __shared__ int mine;
+    if (threadIdx.x == 0) mine = atomicAdd(ticket, 1);
+    __syncthreads();
+    const int vb = mine;
+    const long long base = (long long)vb * kScanBlock + (long long)threadIdx.x * kScanPer;
+    int v[kScanPer];
+    long long sum = 0;
+#pragma unroll
+    for (int j = 0; j < kScanPer; ++j) {
+        v[j] = base + j < n ? in((int)(base + j)) : 0;
+        sum += v[j];
+    }
+    long long ex = 0, agg = 0;
+    BS().exclusive_scan(sum, ex, 0ll, agg, st, rocprim::plus<long long>());
+    if (threadIdx.x == 0) {
+        const auto put = [&](long long x, unsigned long long kind) {
+            __hip_atomic_store(&state[vb], (unsigned long long)x << 2 | kind, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        };
+        long long sofar = 0;
+        if (vb > 0) {
+            put(agg, 1);
+            for (int j = vb - 1;; --j) {
+                unsigned long long w;
+                while (!(w = __hip_atomic_load(&state[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)))
+                    __builtin_amdgcn_s_sleep(1);
+                sofar += (long long)(w >> 2);
+                if (w & 2) break;
+            }
+        }
+        put(sofar + agg, 2);
+        before = sofar;
+        if ((long long)(vb + 1) * kScanBlock >= n) {     // the last workgroup
+            *total = sofar + agg;
+            out[n] = (int)min(sofar + agg, (long long)INT_MAX);
+        }
+    }
+    __syncthreads();
+    long long o = before + ex;
+#pragma unroll
+    for (int j = 0; j < kScanPer; ++j) {
+        if (base + j < n) out[base + j] = (int)min(o, (long long)INT_MAX);
+        o += v[j];
+    }
+}
+inline size_t scan_state_bytes(long long n) { return sizeof(unsigned long long) * (size_t)((n + kScanBlock - 1) / kScanBlock); }
+
+struct IntAt {
+    const int *p;
+    __device__ int operator()(int i) const { return p[i]; }
+};
+
+// ---- 3. the tiles -------------------------------------------------------------
 template <typename V>
 __device__ __forceinline__ V add_round(V a, V b)
 {
@@ -136,30 +478,131 @@ __device__ __forceinline__ V add_round(V a, V b)
     else return a + b;
 }
 
-// one thread per run (distinct column of a block)
-template <typename V>
-__global__ void fill_kernel(const unsigned long long *__restrict__ key, const int *__restrict__ ent,
-                            const uint8_t *__restrict__ lrow, const V *__restrict__ val,
-                            const int *__restrict__ run_start, int nruns, long long n, int cbits, int bm, int bn,
-                            int words, const int *__restrict__ tile_ptr, const int *__restrict__ dstart,
-                            int *__restrict__ cnt, V *__restrict__ dense, unsigned long long *__restrict__ bitmap)
+typedef uint32_t tu4 __attribute__((ext_vector_type(4), may_alias));
+
+// Wave u < tilem: the tiles of row-block u if it has at most kSmall entries;
+// wave tilem + k: the tiles that start in unit k.  BM, BN: the class's tile
+// shape, or 0 with any shape in bm_, bn_.
+// A wave stages a window of tiles in 4 KB of LDS (one tile at least: 8 KB
+// for the widest generic shape) -- enough for 16 tiles of 256 bytes, the
+// most that two 64-entry steps of distinct columns reach -- so eight
+// workgroups of four waves fit on a CU.
+template <typename V, int BM, int BN>
+__global__ __launch_bounds__(kThreads) void fill_kernel(const int *__restrict__ ptr, const int *__restrict__ idx,
+                                                        const V *__restrict__ val, int rows, int nnz, int bm_, int bn_,
+                                                        int tilem, const unsigned *__restrict__ words,
+                                                        const int *__restrict__ tile_ptr,
+                                                        const Unit *__restrict__ units, int nunits, int tilenum,
+                                                        int *__restrict__ colidx, int *__restrict__ tile_nnz,
+                                                        V *__restrict__ dense, unsigned long long *__restrict__ bitmap)
 {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nruns) return;
-    const long long i0 = run_start[r];
-    const long long i1 = r + 1 < nruns ? run_start[r + 1] : n;
-    const int b = (int)(key[i0] >> cbits);
-    const int rank = r - dstart[b];
-    const int tile = tile_ptr[b] + rank / bn, col = rank % bn;
-    V *tv = dense + (size_t)tile * bm * bn;
-    unsigned long long *tb = bitmap + (size_t)tile * words;
-    for (long long i = i0; i < i1; ++i) {
-        const int e = ent[i];
-        const int slot = lrow[e] * bn + col;
-        atomicOr(&tb[slot / 64], 1ull << (slot % 64));
-        tv[slot] = add_round(tv[slot], val[e]);
+    const int bm = BM ? BM : bm_, bn = BN ? BN : bn_;
+    constexpr int kStage = BM ? 4096 : 8192;
+    constexpr int kTiles = 16;
+    constexpr int kMapWords = BM && BN ? (BM * BN + 63) / 64 * (BM * BN * (int)sizeof(V) >= kStage ? 1 : kTiles) : 64;
+    __shared__ __attribute__((aligned(16))) char stage_all[kThreads / 64][kStage];
+    __shared__ unsigned long long map_all[kThreads / 64][kMapWords];
+    __shared__ int row_all[kThreads / 64][64];
+    const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const long long u = (long long)blockIdx.x * (kThreads / 64) + wid;
+    if (u >= (long long)tilem + nunits) return;
+    if (u == 0 && lane == 0) tile_nnz[tilenum] = nnz;
+    Unit un{(int)u, 0, 0, 0};
+    if (u >= tilem) un = units[u - tilem];
+    const int b = un.b;
+    int s, n;
+    block_range(ptr, rows, nnz, bm, tilem, b, s, n);
+    if (n == 0 || (u < tilem && n > kSmall)) return;
+    const int t0 = tile_ptr[b], nt = tile_ptr[b + 1] - t0;
+    // the tiles whose first column starts here
+    const int tb = (un.rank0 + bn - 1) / bn;
+    const int te = (long long)un.p0 + kSmall >= n ? nt : min(nt, (un.rank1 + bn - 1) / bn);
+    if (tb >= te) return;
+    const int slots = bm * bn, mw = (slots + 63) / 64;
+    const int tile_bytes = slots * (int)sizeof(V);       // a multiple of 16: bm is a multiple of 8
+    const int wt = max(1, min(min(kTiles, kStage / tile_bytes), kMapWords / mw));
+    char *stage = stage_all[wid];
+    unsigned long long *map = map_all[wid];
+    int *rowoff = row_all[wid];
+    // first entry of each row after the first; rows past the end never match
+    if (lane < bm) {
+        const long long r = (long long)b * bm + lane;
+        rowoff[lane] = r < rows ? ptr[r] - s : 0x7fffffff;
     }
-    atomicAdd(&cnt[tile], (int)(i1 - i0));
+    auto row_of = [&](int i) {             // the last row that starts at or before entry i
+        int lo = 0;
+        for (int d = bm / 2; d >= 1; d /= 2)
+            if (rowoff[lo + d] <= i) lo += d;
+        return lo;
+    };
+    int p = un.p0, rk = un.rank0;
+    for (int w0 = tb; w0 < te; w0 += wt) {
+        const int w1 = min(w0 + wt, te), nw = w1 - w0;
+        for (int k = lane; k < nw * tile_bytes / 16; k += 64) ((tu4 *)stage)[k] = tu4{0u, 0u, 0u, 0u};
+        for (int k = lane; k < nw * mw; k += 64) map[k] = 0ull;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        for (;;) {
+            const int q = p + lane;
+            const bool in = q < n;
+            const unsigned w = in ? words[s + q] : 0u;
+            const int i = (int)(w & ~kHead);
+            const unsigned long long hm = __ballot(in && (w & kHead));
+            const int rank = rk + __popcll(hm & (2ull << lane) - 1ull) - 1;
+            const int tile = rank >= 0 ? (int)((unsigned)rank / (unsigned)bn) : 0;
+            const bool act = in && tile < w1;
+            const unsigned long long am = __ballot(act);
+            const int row = row_of(i);
+            // the entries before and after this one in sorted order
+            unsigned wb = __shfl_up(w, 1), wa = __shfl_down(w, 1);
+            int rb = __shfl_up(row, 1), ra = __shfl_down(row, 1);
+            if (lane == 0 && q > 0) {
+                wb = words[s + q - 1];
+                rb = row_of((int)(wb & ~kHead));
+            }
+            bool more = q + 1 < n;
+            if (lane == 63 && more) {
+                wa = words[s + q + 1];
+                ra = row_of((int)(wa & ~kHead));
+            }
+            if (act && tile >= w0) {
+                const bool head = (w & kHead) != 0;
+                const int col = rank - tile * bn;
+                if (head) {
+                    colidx[(size_t)t0 * bn + rank] = idx[s + i];
+                    if (col == 0) tile_nnz[t0 + tile] = s + q;
+                }
+                if (head || rb != row) {   // the first entry of its slot
+                    V v = add_round((V)0, val[s + i]);
+                    more = more && !(wa & kHead) && ra == row;
+                    for (int k = q + 1; more;) {
+                        v = add_round(v, val[s + (int)(wa & ~kHead)]);
+                        more = ++k < n;
+                        if (more) {
+                            wa = words[s + k];
+                            more = !(wa & kHead) && row_of((int)(wa & ~kHead)) == row;
+                        }
+                    }
+                    const int slot = row * bn + col, tl = tile - w0;
+                    ((V *)stage)[tl * slots + slot] = v;
+                    atomicOr((unsigned *)map + 2 * (tl * mw) + slot / 32, 1u << (slot & 31));
+                }
+            }
+            const int na = __popcll(am);
+            p += na;
+            rk += __popcll(hm & am);
+            if (na < 64) break;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        tu4 *out = (tu4 *)((char *)dense + (size_t)(t0 + w0) * tile_bytes);
+        for (int k = lane; k < nw * tile_bytes / 16; k += 64) out[k] = ((const tu4 *)stage)[k];
+        for (int k = lane; k < nw * mw; k += 64) bitmap[(size_t)(t0 + w0) * mw + k] = map[k];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+    if (te == nt) {
+        // the block's last tile repeats its last column
+        const int last = idx[s + (int)(words[s + n - 1] & ~kHead)];
+        for (long long k = rk + lane; k < (long long)nt * bn; k += 64) colidx[(size_t)t0 * bn + k] = last;
+    }
 }
 
 // ---- bitmap-packed A -------------------------------------------------------
@@ -341,14 +784,52 @@ struct DevBufs {
         if (e_ != hipSuccess) return (int)e_;       \
     } while (0)
 
-template <typename T>
-int scan_excl(Scratch &tmp, const T *in, T *out, size_t n, hipStream_t s)
+// One allocation cut into 256-byte aligned pieces.
+struct Carve {
+    size_t bytes = 0;
+    size_t add(size_t n)
+    {
+        const size_t at = bytes;
+        bytes += (n + 255) / 256 * 256;
+        return at;
+    }
+};
+
+template <typename F>
+int launch_scan(F in, int n, int *out, unsigned long long *state, int *ticket, long long *total, hipStream_t s)
 {
+    scan_kernel<<<(unsigned)(((long long)n + kScanBlock - 1) / kScanBlock), kThreads, 0, s>>>(in, n, out, state, ticket,
+                                                                                              total);
+    return (int)hipGetLastError();
+}
+
+// Sorts the entries of the `nh` huge blocks (`entries` in all) and completes
+// their words, units and tile counts.
+int sort_huge(const int *d_ptr, const int *d_idx, int rows, int nnz, int bm, int bn, int tilem, int cbits, int colA,
+              const Big *huge, unsigned nh, size_t entries, unsigned *words, Unit *units, int *nt, Counters *cnt,
+              hipStream_t s)
+{
+    const int bits = cbits + bits_for(nh);
+    unsigned long long *key = nullptr;
+    unsigned *pos = nullptr;
     size_t need = 0;
-    TCHK(rocprim::exclusive_scan(nullptr, need, in, out, T(0), n, rocprim::plus<T>(), s));
-    TCHK(tmp.grow(need));
-    TCHK(rocprim::exclusive_scan(tmp.p, need, in, out, T(0), n, rocprim::plus<T>(), s));
-    return 0;
+    TCHK(rocprim::radix_sort_pairs(nullptr, need, key, key, pos, pos, entries, 0, bits, s));
+    Carve c;
+    const size_t k0 = c.add(8 * entries), k1 = c.add(8 * entries), p0 = c.add(4 * entries), p1 = c.add(4 * entries);
+    const size_t t0 = c.add(need);
+    DevBufs db;
+    char *w = nullptr;
+    TCHK(db.get(&w, c.bytes));
+    const dim3 grid(nh, kHugeY);
+    huge_keys_kernel<<<grid, kThreads, 0, s>>>(d_ptr, d_idx, rows, nnz, bm, tilem, cbits, colA, huge,
+                                               (unsigned long long *)(w + k0), (unsigned *)(w + p0), cnt);
+    TCHK(rocprim::radix_sort_pairs(w + t0, need, (unsigned long long *)(w + k0), (unsigned long long *)(w + k1),
+                                   (unsigned *)(w + p0), (unsigned *)(w + p1), entries, 0, bits, s));
+    huge_words_kernel<<<grid, kThreads, 0, s>>>(d_ptr, rows, nnz, bm, tilem, huge, (unsigned long long *)(w + k1),
+                                                (unsigned *)(w + p1), words, units);
+    huge_ranks_kernel<<<nh, kThreads, 0, s>>>(d_ptr, rows, nnz, bm, bn, tilem, huge, units, nt);
+    TCHK(hipGetLastError());
+    return (int)hipStreamSynchronize(s);       // the buffers go
 }
 
 int tile_create_device(tsp_dev_tiles *out, int rows, int colA, long long nnz, const int *d_ptr, const int *d_idx,
@@ -378,78 +859,88 @@ int tile_create_device(tsp_dev_tiles *out, int rows, int colA, long long nnz, co
         return (int)hipStreamSynchronize(s);
     }
     const int cbits = bits_for(colA);
-    const int bbits = bits_for(tilem);
-    const size_t n = (size_t)nnz;
+    const unsigned cmask = (unsigned)((1ull << cbits) - 1ull);
+    const int n = (int)nnz;
+    // every medium block holds more than kSmall entries, every huge one more
+    // than kMedium, and a block of n of them has at most 2 n / kSmall units
+    const int medium_cap = n / kSmall + 1, huge_cap = n / kMedium + 1, unit_cap = 2 * (n / kSmall) + 2;
+    const size_t state_bytes = scan_state_bytes(tilem);
+    Carve cv;
+    const size_t o_cnt = cv.add(sizeof(Counters)), o_state = cv.add(state_bytes);
+    const size_t zeroed = cv.bytes;
+    const size_t o_nt = cv.add(4 * (size_t)tilem), o_medium = cv.add(sizeof(Big) * (size_t)medium_cap);
+    const size_t o_huge = cv.add(sizeof(Big) * (size_t)huge_cap), o_units = cv.add(sizeof(Unit) * (size_t)unit_cap);
+    const size_t o_words = cv.add(4 * (size_t)n);
     DevBufs db;
-    Scratch tmp;
-    unsigned long long *key = nullptr, *key2 = nullptr;
-    int *ent = nullptr, *ent2 = nullptr, *flag = nullptr, *run = nullptr, *run_start = nullptr, *dcols = nullptr;
-    int *bptr = nullptr, *dstart = nullptr, *nt = nullptr, *bad = nullptr;
-    uint8_t *lrow = nullptr;
-    TCHK(db.get(&key, n * 8));
-    TCHK(db.get(&key2, n * 8));
-    TCHK(db.get(&ent, n * 4));
-    TCHK(db.get(&ent2, n * 4));
-    TCHK(db.get(&lrow, n));
-    TCHK(db.get(&flag, (n + 1) * 4));
-    TCHK(db.get(&run, (n + 1) * 4));
-    TCHK(db.get(&run_start, n * 4));
-    TCHK(db.get(&dcols, n * 4));
-    TCHK(db.get(&bptr, ((size_t)tilem + 1) * 4));
-    TCHK(db.get(&dstart, ((size_t)tilem + 1) * 4));
-    TCHK(db.get(&nt, ((size_t)tilem + 1) * 4));
-    TCHK(db.get(&bad, 4));
-    TCHK(hipMemsetAsync(bad, 0, 4, s));
-    block_ptr_kernel<<<nblocks(tilem + 1), kThreads, 0, s>>>(d_ptr, rows, tilem, BM, bptr);
-    key_kernel<<<nblocks(nnz), kThreads, 0, s>>>(d_ptr, d_idx, rows, nnz, BM, cbits, colA, key, ent, lrow, bad);
-    // 1. stable sort by (block, column)
-    size_t need = 0;
-    TCHK(rocprim::radix_sort_pairs(nullptr, need, key, key2, ent, ent2, n, 0, cbits + bbits, s));
-    TCHK(tmp.grow(need));
-    TCHK(rocprim::radix_sort_pairs(tmp.p, need, key, key2, ent, ent2, n, 0, cbits + bbits, s));
-    // 2. runs
-    TCHK(hipMemsetAsync(flag + n, 0, 4, s));
-    head_kernel<<<nblocks(nnz), kThreads, 0, s>>>(key2, nnz, flag);
-    if (int st = scan_excl(tmp, flag, run, n + 1, s)) return st;
-    run_scatter_kernel<<<nblocks(nnz), kThreads, 0, s>>>(key2, flag, run, nnz, (1u << cbits) - 1u, run_start,
-                                                        dcols);
-    // 3. tiles per block, tile_ptr
-    TCHK(hipMemsetAsync(nt + tilem, 0, 4, s));
-    block_runs_kernel<<<nblocks(tilem), kThreads, 0, s>>>(bptr, run, tilem, BN, dstart, nt);
-    int nruns = 0;
-    TCHK(hipMemcpyAsync(&nruns, run + n, 4, hipMemcpyDeviceToHost, s));
-    TCHK(hipMemcpyAsync(dstart + tilem, run + n, 4, hipMemcpyDeviceToDevice, s));
-    if (int st = scan_excl(tmp, nt, out->d_tile_ptr, (size_t)tilem + 1, s)) return st;
-    int tilenum = 0, nbad = 0;
-    TCHK(hipMemcpyAsync(&tilenum, out->d_tile_ptr + tilem, 4, hipMemcpyDeviceToHost, s));
-    TCHK(hipMemcpyAsync(&nbad, bad, 4, hipMemcpyDeviceToHost, s));
-    TCHK(hipStreamSynchronize(s));
-    if (nbad) return TSP_EINVAL;        // a column outside [0, colA)
-    // every tile holds at least one entry, so tilenum <= nnz < 2^31
+    char *w = nullptr;
+    TCHK(db.get(&w, cv.bytes));
+    Counters *cnt = (Counters *)(w + o_cnt);
+    unsigned long long *state = (unsigned long long *)(w + o_state);
+    int *nt = (int *)(w + o_nt);
+    Big *medium = (Big *)(w + o_medium), *huge = (Big *)(w + o_huge);
+    Unit *units = (Unit *)(w + o_units);
+    unsigned *words = (unsigned *)(w + o_words);
+    TCHK(hipMemsetAsync(w, 0, zeroed, s));
+    // 1. sorted entries, tiles per block
+    const unsigned wave_blocks = nblocks((long long)tilem * 64);
+    if (cbits + kSmallBits <= 32)
+        sort_blocks_kernel<unsigned><<<wave_blocks, kThreads, 0, s>>>(d_ptr, d_idx, rows, n, BM, BN, tilem, cmask, colA,
+                                                                      words, nt, medium, medium_cap, huge, huge_cap,
+                                                                      unit_cap, cnt);
+    else
+        sort_blocks_kernel<unsigned long long><<<wave_blocks, kThreads, 0, s>>>(
+            d_ptr, d_idx, rows, n, BM, BN, tilem, cmask, colA, words, nt, medium, medium_cap, huge, huge_cap, unit_cap,
+            cnt);
+    if (n > kSmall)
+        sort_medium_kernel<<<(unsigned)(medium_cap < 512 ? medium_cap : 512), kMediumThreads, 0, s>>>(
+            d_ptr, d_idx, rows, n, BM, BN, tilem, cmask, colA, words, nt, medium, medium_cap, units, cnt);
+    TCHK(hipGetLastError());
+    // 2. tile_ptr
+    Counters h;
+    for (int pass = 0;; ++pass) {
+        if (int st = launch_scan(IntAt{nt}, tilem, out->d_tile_ptr, state, &cnt->ticket, &cnt->total, s)) return st;
+        TCHK(hipMemcpyAsync(&h, cnt, sizeof h, hipMemcpyDeviceToHost, s));
+        TCHK(hipStreamSynchronize(s));
+        if (h.bad) return TSP_EINVAL;       // a column outside [0, colA)
+        const size_t entries = (size_t)(h.huge & ((1ull << 40) - 1ull));
+        if (entries == 0 || pass) break;
+        if (int st = sort_huge(d_ptr, d_idx, rows, n, BM, BN, tilem, cbits, colA, huge, (unsigned)(h.huge >> 40), entries,
+                               words, units, nt, cnt, s))
+            return st;
+        TCHK(hipMemsetAsync(state, 0, state_bytes, s));
+        TCHK(hipMemsetAsync(&cnt->ticket, 0, sizeof(int), s));
+    }
+    // every tile holds at least one entry
+    if (h.total > nnz) return TSP_EINVAL;
+    const int tilenum = (int)h.total;
     out->tilenum = tilenum;
     const size_t tn = (size_t)tilenum;
     TCHK(hipMalloc(&out->d_tile_colidx, 4 * tn * BN));
     TCHK(hipMalloc(&out->d_tile_nnz, 4 * (tn + 1)));
     TCHK(hipMalloc(&out->d_val, vs * tn * BM * BN));
     TCHK(hipMalloc((void **)&out->d_bitmap, 8 * tn * out->bitmap_words));
-    int *cnt = nullptr;
-    TCHK(db.get(&cnt, 4 * (tn + 1)));
-    TCHK(hipMemsetAsync(cnt, 0, 4 * (tn + 1), s));
-    TCHK(hipMemsetAsync(out->d_val, 0, vs * tn * BM * BN, s));
-    TCHK(hipMemsetAsync(out->d_bitmap, 0, 8 * tn * out->bitmap_words, s));
-    colidx_kernel<<<tilem, kThreads, 0, s>>>(out->d_tile_ptr, dstart, dcols, BN, out->d_tile_colidx);
-    // 4. values, counts, bitmaps
-    if (prec == TSP_PREC_FP16)
-        fill_kernel<_Float16><<<nblocks(nruns), kThreads, 0, s>>>(
-            key2, ent2, lrow, (const _Float16 *)d_val, run_start, nruns, nnz, cbits, BM, BN, out->bitmap_words,
-            out->d_tile_ptr, dstart, cnt, (_Float16 *)out->d_val, (unsigned long long *)out->d_bitmap);
-    else
-        fill_kernel<float><<<nblocks(nruns), kThreads, 0, s>>>(
-            key2, ent2, lrow, (const float *)d_val, run_start, nruns, nnz, cbits, BM, BN, out->bitmap_words,
-            out->d_tile_ptr, dstart, cnt, (float *)out->d_val, (unsigned long long *)out->d_bitmap);
+    // 3. the tiles
+    const unsigned fill_blocks = nblocks(((long long)tilem + h.nunits) * 64);
+    const auto fill = [&](auto kernel, auto *v) {
+        kernel<<<fill_blocks, kThreads, 0, s>>>(d_ptr, d_idx, v, rows, n, BM, BN, tilem, words, out->d_tile_ptr, units,
+                                                h.nunits, tilenum, out->d_tile_colidx, out->d_tile_nnz,
+                                                (std::remove_const_t<std::remove_pointer_t<decltype(v)>> *)out->d_val,
+                                                (unsigned long long *)out->d_bitmap);
+    };
+    if (prec == TSP_PREC_FP16) {
+        const _Float16 *v = (const _Float16 *)d_val;
+        if (BM == 8 && BN == 16) fill(fill_kernel<_Float16, 8, 16>, v);
+        else if (BM == 16 && BN == 16) fill(fill_kernel<_Float16, 16, 16>, v);
+        else if (BM == 64 && BN == 32) fill(fill_kernel<_Float16, 64, 32>, v);
+        else fill(fill_kernel<_Float16, 0, 0>, v);
+    } else {
+        const float *v = (const float *)d_val;
+        if (BM == 8 && BN == 8) fill(fill_kernel<float, 8, 8>, v);
+        else if (BM == 16 && BN == 8) fill(fill_kernel<float, 16, 8>, v);
+        else if (BM == 64 && BN == 16) fill(fill_kernel<float, 64, 16>, v);
+        else fill(fill_kernel<float, 0, 0>, v);
+    }
     TCHK(hipGetLastError());
-    // 5. tile_nnz
-    if (int st = scan_excl(tmp, cnt, out->d_tile_nnz, tn + 1, s)) return st;
     return (int)hipStreamSynchronize(s);
 }
 
