@@ -84,9 +84,14 @@ int tsp_kernel_probe(int bm, int prec, int colB_p, tsp_kernel_info *out);
  * (status TSP_OK) when the clock cannot be read. */
 int tsp_gpu_clock_mhz(int device_id, unsigned *mhz, unsigned *max_mhz);
 
-/* Memory and copies (hipMalloc / hipMemcpy / hipMemset wrappers). */
+/* Memory and copies (hipMalloc / hipMemcpy / hipMemset wrappers).  tsp_free
+ * waits for the device, as hipFree does, and keeps the block for a later
+ * tsp_malloc of about its size on that device (whole hipMalloc allocations,
+ * idle ones at most 1/32 of the device's memory; a block may also be passed
+ * to hipFree).  tsp_mem_trim gives every idle block back to the system. */
 int tsp_malloc(void **ptr, size_t bytes);
 int tsp_free(void *ptr);
+int tsp_mem_trim(void);
 int tsp_memcpy_h2d(void *dst, const void *src, size_t bytes);
 int tsp_memcpy_d2h(void *dst, const void *src, size_t bytes);
 int tsp_memcpy_h2d_async(void *dst, const void *src, size_t bytes, void *stream);

@@ -139,6 +139,7 @@ HIP_SYMBOLS = {
     "tsp_gpu_clock_mhz": (C.c_int, [C.c_int, C.POINTER(C.c_uint), C.POINTER(C.c_uint)]),
     "tsp_malloc": (C.c_int, [C.POINTER(C.c_void_p), C.c_size_t]),
     "tsp_free": (C.c_int, [_P]),
+    "tsp_mem_trim": (C.c_int, []),
     "tsp_memcpy_h2d": (C.c_int, [_P, _P, C.c_size_t]),
     "tsp_memcpy_d2h": (C.c_int, [_P, _P, C.c_size_t]),
     "tsp_memcpy_h2d_async": (C.c_int, [_P, _P, C.c_size_t, _P]),

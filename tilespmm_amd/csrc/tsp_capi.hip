@@ -150,18 +150,6 @@ int tsp_gpu_clock_mhz(int device_id, unsigned *mhz, unsigned *max_mhz)
     return TSP_OK;
 }
 
-int tsp_malloc(void **ptr, size_t bytes)
-{
-    if (!ptr) return TSP_EINVAL;
-    *ptr = nullptr;
-    if (bytes == 0) return TSP_OK;
-    const hipError_t e = hipMalloc(ptr, bytes);
-    // a failed allocation must not surface later as the error of an
-    // unrelated launch (launches report hipGetLastError)
-    if (e != hipSuccess) (void)hipGetLastError();
-    return (int)e;
-}
-int tsp_free(void *ptr) { return ptr ? (int)hipFree(ptr) : TSP_OK; }
 int tsp_memcpy_h2d(void *dst, const void *src, size_t bytes)
 {
     return bytes ? (int)hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice) : TSP_OK;

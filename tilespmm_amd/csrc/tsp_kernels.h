@@ -152,6 +152,12 @@ int launch_gather(const void *table, size_t table_bytes, int row_bytes, int iter
 int launch_stream_gather(const void *table, long long nrows, int row_bytes, const int *idx, long long n, void *sink,
                          hipStream_t s);
 
+// Device memory through the pool of tsp_mem.hip (tsp_malloc / tsp_free).
+// waited: the caller has waited for every stream that used the block;
+// otherwise dev_free waits for the block's device.
+int dev_alloc(void **ptr, size_t bytes);
+int dev_free(void *ptr, bool waited);
+
 // Address of the allocation-free entry points' `scratch` array on the current
 // device (looked up once per device; tsp_device_init calls it).
 int scratch_init_current_device(int **ptr);

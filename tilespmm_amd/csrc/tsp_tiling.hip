@@ -741,47 +741,33 @@ __global__ void pack_tail_kernel(int *__restrict__ vptr, int tilenum, const int 
     if ((int)threadIdx.x < nz && (long long)total + threadIdx.x < cap) pval[(long long)total + threadIdx.x] = V(0);
 }
 
-struct Scratch {
-    void *p = nullptr;
-    size_t bytes = 0;
-    hipError_t grow(size_t n)
-    {
-        if (n <= bytes) return hipSuccess;
-        if (p) (void)hipFree(p);
-        bytes = 0;
-        hipError_t e = hipMalloc(&p, n ? n : 16);
-        if (e == hipSuccess) bytes = n;
-        return e;
-    }
-    ~Scratch()
-    {
-        if (p) (void)hipFree(p);
-    }
-};
-
-// device buffers freed at scope exit
+// Device buffers of one call, all used on `stream` only: given back at scope
+// exit, once the stream has drained.
 struct DevBufs {
-    void *p[16] = {};
+    hipStream_t stream;
+    void *p[4] = {};
     int n = 0;
+    explicit DevBufs(hipStream_t s) : stream(s) {}
     template <typename T>
-    hipError_t get(T **out, size_t bytes)
+    int get(T **out, size_t bytes)
     {
         void *q = nullptr;
-        hipError_t e = hipMalloc(&q, bytes ? bytes : 16);
-        if (e == hipSuccess) p[n++] = q;
+        const int st = tsp::dev_alloc(&q, bytes);
+        if (st == 0) p[n++] = q;
         *out = (T *)q;
-        return e;
+        return st;
     }
     ~DevBufs()
     {
-        for (int i = 0; i < n; ++i) (void)hipFree(p[i]);
+        const bool waited = n > 0 && hipStreamSynchronize(stream) == hipSuccess;
+        for (int i = 0; i < n; ++i) (void)tsp::dev_free(p[i], waited);
     }
 };
 
 #define TCHK(x)                                     \
     do {                                            \
-        hipError_t e_ = (x);                        \
-        if (e_ != hipSuccess) return (int)e_;       \
+        const int e_ = (int)(x);                    \
+        if (e_ != 0) return e_;                     \
     } while (0)
 
 // One allocation cut into 256-byte aligned pieces.
@@ -817,7 +803,7 @@ int sort_huge(const int *d_ptr, const int *d_idx, int rows, int nnz, int bm, int
     Carve c;
     const size_t k0 = c.add(8 * entries), k1 = c.add(8 * entries), p0 = c.add(4 * entries), p1 = c.add(4 * entries);
     const size_t t0 = c.add(need);
-    DevBufs db;
+    DevBufs db(s);
     char *w = nullptr;
     TCHK(db.get(&w, c.bytes));
     const dim3 grid(nh, kHugeY);
@@ -828,8 +814,7 @@ int sort_huge(const int *d_ptr, const int *d_idx, int rows, int nnz, int bm, int
     huge_words_kernel<<<grid, kThreads, 0, s>>>(d_ptr, rows, nnz, bm, tilem, huge, (unsigned long long *)(w + k1),
                                                 (unsigned *)(w + p1), words, units);
     huge_ranks_kernel<<<nh, kThreads, 0, s>>>(d_ptr, rows, nnz, bm, bn, tilem, huge, units, nt);
-    TCHK(hipGetLastError());
-    return (int)hipStreamSynchronize(s);       // the buffers go
+    return (int)hipGetLastError();
 }
 
 int tile_create_device(tsp_dev_tiles *out, int rows, int colA, long long nnz, const int *d_ptr, const int *d_idx,
@@ -847,14 +832,14 @@ int tile_create_device(tsp_dev_tiles *out, int rows, int colA, long long nnz, co
     const int tilem = (rows + BM - 1) / BM;
     out->tilem = tilem;
     const size_t vs = prec == TSP_PREC_FP16 ? 2 : 4;
-    TCHK(hipMalloc(&out->d_tile_ptr, sizeof(int) * ((size_t)tilem + 1)));
+    TCHK(tsp::dev_alloc((void **)&out->d_tile_ptr, sizeof(int) * ((size_t)tilem + 1)));
     if (tilem == 0 || nnz == 0) {
         // no entries: every row-block has zero tiles
         TCHK(hipMemsetAsync(out->d_tile_ptr, 0, sizeof(int) * ((size_t)tilem + 1), s));
-        TCHK(hipMalloc(&out->d_tile_colidx, 16));
-        TCHK(hipMalloc(&out->d_val, 16));
-        TCHK(hipMalloc((void **)&out->d_bitmap, 16));
-        TCHK(hipMalloc(&out->d_tile_nnz, sizeof(int)));
+        TCHK(tsp::dev_alloc((void **)&out->d_tile_colidx, 16));
+        TCHK(tsp::dev_alloc((void **)&out->d_val, 16));
+        TCHK(tsp::dev_alloc((void **)&out->d_bitmap, 16));
+        TCHK(tsp::dev_alloc((void **)&out->d_tile_nnz, sizeof(int)));
         TCHK(hipMemsetAsync(out->d_tile_nnz, 0, sizeof(int), s));
         return (int)hipStreamSynchronize(s);
     }
@@ -871,7 +856,7 @@ int tile_create_device(tsp_dev_tiles *out, int rows, int colA, long long nnz, co
     const size_t o_nt = cv.add(4 * (size_t)tilem), o_medium = cv.add(sizeof(Big) * (size_t)medium_cap);
     const size_t o_huge = cv.add(sizeof(Big) * (size_t)huge_cap), o_units = cv.add(sizeof(Unit) * (size_t)unit_cap);
     const size_t o_words = cv.add(4 * (size_t)n);
-    DevBufs db;
+    DevBufs db(s);
     char *w = nullptr;
     TCHK(db.get(&w, cv.bytes));
     Counters *cnt = (Counters *)(w + o_cnt);
@@ -915,10 +900,10 @@ int tile_create_device(tsp_dev_tiles *out, int rows, int colA, long long nnz, co
     const int tilenum = (int)h.total;
     out->tilenum = tilenum;
     const size_t tn = (size_t)tilenum;
-    TCHK(hipMalloc(&out->d_tile_colidx, 4 * tn * BN));
-    TCHK(hipMalloc(&out->d_tile_nnz, 4 * (tn + 1)));
-    TCHK(hipMalloc(&out->d_val, vs * tn * BM * BN));
-    TCHK(hipMalloc((void **)&out->d_bitmap, 8 * tn * out->bitmap_words));
+    TCHK(tsp::dev_alloc((void **)&out->d_tile_colidx, 4 * tn * BN));
+    TCHK(tsp::dev_alloc((void **)&out->d_tile_nnz, 4 * (tn + 1)));
+    TCHK(tsp::dev_alloc((void **)&out->d_val, vs * tn * BM * BN));
+    TCHK(tsp::dev_alloc((void **)&out->d_bitmap, 8 * tn * out->bitmap_words));
     // 3. the tiles
     const unsigned fill_blocks = nblocks(((long long)tilem + h.nunits) * 64);
     const auto fill = [&](auto kernel, auto *v) {
@@ -1045,19 +1030,16 @@ int tsp_tiles_pack_device(int tilenum, int bm, int bn, int prec, const void *d_v
     hipStream_t s = (hipStream_t)stream;
     const int words = (bm * bn + 63) / 64;
     int *vptr = nullptr, *cnt = nullptr;
-    Scratch tmp;
+    char *tmp = nullptr;
+    DevBufs db(s);
     // the counts, then (8-byte aligned) their 64-bit total
     const size_t cnt_bytes = (sizeof(int) * ((size_t)tilenum + 1) + 7) / 8 * 8;
-    TCHK(hipMalloc(&cnt, cnt_bytes + sizeof(unsigned long long)));
+    TCHK(db.get(&cnt, cnt_bytes + sizeof(unsigned long long)));
     unsigned long long *total64 = (unsigned long long *)((char *)cnt + cnt_bytes);
-    struct FreeCnt {
-        int *p;
-        ~FreeCnt() { (void)hipFree(p); }
-    } fc{cnt};
-    hipError_t e = hipMalloc(&vptr, sizeof(int) * ((size_t)tilenum + 1));
-    if (e != hipSuccess) return (int)e;
+    TCHK(tsp::dev_alloc((void **)&vptr, sizeof(int) * ((size_t)tilenum + 1)));
+    hipError_t e = hipSuccess;
     auto fail = [&](int st) {
-        (void)hipFree(vptr);
+        (void)tsp::dev_free(vptr, false);
         return st;
     };
     if ((e = hipMemsetAsync(cnt + tilenum, 0, sizeof(int), s)) != hipSuccess) return fail((int)e);
@@ -1078,8 +1060,8 @@ int tsp_tiles_pack_device(int tilenum, int bm, int bn, int prec, const void *d_v
     if ((e = rocprim::exclusive_scan(nullptr, need, cnt, vptr, 0, (size_t)tilenum + 1, rocprim::plus<int>(), s)) !=
         hipSuccess)
         return fail((int)e);
-    if ((e = tmp.grow(need)) != hipSuccess) return fail((int)e);
-    if ((e = rocprim::exclusive_scan(tmp.p, need, cnt, vptr, 0, (size_t)tilenum + 1, rocprim::plus<int>(), s)) !=
+    if (const int st = db.get(&tmp, need)) return fail(st);
+    if ((e = rocprim::exclusive_scan(tmp, need, cnt, vptr, 0, (size_t)tilenum + 1, rocprim::plus<int>(), s)) !=
         hipSuccess)
         return fail((int)e);
     const int total = (int)total_u;
@@ -1087,9 +1069,9 @@ int tsp_tiles_pack_device(int tilenum, int bm, int bn, int prec, const void *d_v
     // 4 elements of zero padding: the kernels' packed loads may read past the last value
     const size_t vs = prec == TSP_PREC_FP16 ? 2 : 4;
     void *pv = nullptr;
-    if ((e = hipMalloc(&pv, vs * ((size_t)total + 4))) != hipSuccess) return fail((int)e);
+    if (const int st = tsp::dev_alloc(&pv, vs * ((size_t)total + 4))) return fail(st);
     if ((e = hipMemsetAsync((char *)pv + vs * (size_t)total, 0, vs * 4, s)) != hipSuccess) {
-        (void)hipFree(pv);
+        (void)tsp::dev_free(pv, false);
         return fail((int)e);
     }
     if (tilenum > 0) {
@@ -1101,7 +1083,7 @@ int tsp_tiles_pack_device(int tilenum, int bm, int bn, int prec, const void *d_v
                 (const uint32_t *)d_val, d_bitmap, vptr, tilenum, words, bm * bn, (uint32_t *)pv, total);
     }
     if ((e = hipGetLastError()) != hipSuccess || (e = hipStreamSynchronize(s)) != hipSuccess) {
-        (void)hipFree(pv);
+        (void)tsp::dev_free(pv, false);
         return fail((int)e);
     }
     *d_pval = pv;
@@ -1112,11 +1094,12 @@ int tsp_tiles_pack_device(int tilenum, int bm, int bn, int prec, const void *d_v
 int tsp_dev_tiles_free(tsp_dev_tiles *t)
 {
     if (!t) return TSP_OK;
-    (void)hipFree(t->d_tile_ptr);
-    (void)hipFree(t->d_tile_nnz);
-    (void)hipFree(t->d_tile_colidx);
-    (void)hipFree(t->d_val);
-    (void)hipFree(t->d_bitmap);
+    // the first one's wait covers the rest
+    const bool waited = tsp::dev_free(t->d_val, false) == TSP_OK && t->d_val;
+    (void)tsp::dev_free(t->d_tile_ptr, waited);
+    (void)tsp::dev_free(t->d_tile_nnz, waited);
+    (void)tsp::dev_free(t->d_tile_colidx, waited);
+    (void)tsp::dev_free(t->d_bitmap, waited);
     memset(t, 0, sizeof *t);
     return TSP_OK;
 }
