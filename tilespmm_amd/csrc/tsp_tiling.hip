@@ -22,7 +22,7 @@
 //
 // The conversion is bound by memory traffic: it reads the column indices
 // twice, the values once, the 4-byte scratch twice, and writes the tiles
-// once.  RMAT scale 22 (128M entries) to tf32 8-row tiles: 8.9 ms of kernels,
+// once.  RMAT scale 22 (128M entries) to tf32 8-row tiles: 7.5 ms of kernels,
 // against 28 ms for a global radix sort of 8-byte keys over all entries with
 // cleared output arrays filled by one thread per column run.
 #include <cstring>
@@ -84,6 +84,7 @@ struct Counters {
     unsigned long long huge;               // (blocks << 40) + entries of the globally sorted blocks
     long long total;                       // tiles
     int bad;                               // a column outside [0, colA), or row pointers out of order
+    int dups;                              // some row's columns do not ascend: a slot may have several entries
     int nunits, nmedium;
     int ticket;                            // of the chained scan
 };
@@ -153,20 +154,28 @@ __device__ __forceinline__ void bitonic(K (&x)[R], int t, F &&other)
 
 // Sorts the n <= 64 R entries of a block at CSR position s, one wave; writes
 // their sorted words and returns the number of distinct columns.
+// starts: bit i set where a row starts at entry i.
 template <typename K, int R>
 __device__ __forceinline__ int sort_small(const int *__restrict__ idx, int s, int n, unsigned cmask, int colA, int lane,
-                                          unsigned *__restrict__ words, bool &bad)
+                                          const unsigned long long *starts, unsigned *__restrict__ words, bool &bad,
+                                          bool &dups)
 {
     K x[R];
+    int prev = -1;                         // the column before this step's first
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         const int i = r * 64 + lane;
         x[r] = ~(K)0;                      // past every entry
+        int c = 0x7fffffff;
         if (i < n) {
-            const unsigned c = (unsigned)idx[s + i];
-            bad |= c >= (unsigned)colA;
-            x[r] = (K)(c & cmask) << kSmallBits | (unsigned)i;
+            c = idx[s + i];
+            bad |= (unsigned)c >= (unsigned)colA;
+            x[r] = (K)((unsigned)c & cmask) << kSmallBits | (unsigned)i;
         }
+        int before = __shfl_up(c, 1);
+        if (lane == 0) before = prev;
+        dups |= (__ballot(i < n && c <= before) & ~starts[r]) != 0;
+        prev = __builtin_amdgcn_readlane(c, 63);
     }
     bitonic<2, 64 * R>(x, lane, [](const K (&v)[R], K (&y)[R], int d, bool flip) {
 #pragma unroll
@@ -201,8 +210,18 @@ __global__ __launch_bounds__(kThreads) void sort_blocks_kernel(const int *__rest
     block_range(ptr, rows, nnz, bm, tilem, b, s, n);
     s = __builtin_amdgcn_readfirstlane(s);
     n = __builtin_amdgcn_readfirstlane(n);
-    bool bad = false;
+    bool bad = false, dups = false;
     int d = 0;
+    __shared__ unsigned long long starts_all[kThreads / 64][kSmall / 64];
+    unsigned long long *starts = starts_all[threadIdx.x >> 6];
+    if (n > 0 && n <= kSmall) {
+        if (lane < kSmall / 64) starts[lane] = 0ull;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        const long long r = (long long)b * bm + lane;
+        const int at = lane < bm && r < rows ? ptr[r] - s : -1;
+        if (at >= 0 && at < n) atomicOr((unsigned *)starts + (at >> 5), 1u << (at & 31));
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
     if (n > kSmall) {
         if (lane == 0) {
             const int ns = (n + kSmall - 1) / kSmall;
@@ -221,25 +240,42 @@ __global__ __launch_bounds__(kThreads) void sort_blocks_kernel(const int *__rest
             }
         }
     } else if (n > 512) {
-        d = sort_small<K, 16>(idx, s, n, cmask, colA, lane, words, bad);
+        d = sort_small<K, 16>(idx, s, n, cmask, colA, lane, starts, words, bad, dups);
     } else if (n > 256) {
-        d = sort_small<K, 8>(idx, s, n, cmask, colA, lane, words, bad);
+        d = sort_small<K, 8>(idx, s, n, cmask, colA, lane, starts, words, bad, dups);
     } else if (n > 128) {
-        d = sort_small<K, 4>(idx, s, n, cmask, colA, lane, words, bad);
+        d = sort_small<K, 4>(idx, s, n, cmask, colA, lane, starts, words, bad, dups);
     } else if (n > 64) {
-        d = sort_small<K, 2>(idx, s, n, cmask, colA, lane, words, bad);
+        d = sort_small<K, 2>(idx, s, n, cmask, colA, lane, starts, words, bad, dups);
     } else if (n > 0) {
-        d = sort_small<K, 1>(idx, s, n, cmask, colA, lane, words, bad);
+        d = sort_small<K, 1>(idx, s, n, cmask, colA, lane, starts, words, bad, dups);
     }
     if (lane == 0) nt[b] = (d + bn - 1) / bn;
     if (bad) cnt->bad = 1;
+    if (dups) cnt->dups = 1;
+}
+
+// Whether entry i > 0 of a block of CSR position s may share its slot with
+// an earlier one: its column c does not exceed the one before it, and no row
+// starts at it.
+__device__ __forceinline__ bool not_ascending(const int *__restrict__ ptr, const int *__restrict__ idx, int rows, int bm,
+                                              int b, int s, int i, int c)
+{
+    if (i == 0 || c > idx[s + i - 1]) return false;
+    for (int j = 0; j < bm; ++j) {
+        const long long r = (long long)b * bm + j;
+        if (r < rows && ptr[r] - s == i) return false;
+    }
+    return true;
 }
 
 // Sorts one block of at most kMediumThreads * R entries by the workgroup.
 template <int R>
-__device__ __forceinline__ void sort_medium(const int *__restrict__ idx, int s, int n, unsigned cmask, int colA, Big m,
-                                            int bn, unsigned *__restrict__ words, int *__restrict__ nt,
-                                            Unit *__restrict__ units, unsigned long long *lds, int *heads, bool &bad)
+__device__ __forceinline__ void sort_medium(const int *__restrict__ ptr, const int *__restrict__ idx, int rows, int bm,
+                                            int s, int n, unsigned cmask, int colA, Big m, int bn,
+                                            unsigned *__restrict__ words, int *__restrict__ nt,
+                                            Unit *__restrict__ units, unsigned long long *lds, int *heads, bool &bad,
+                                            bool &dups)
 {
     typedef unsigned long long K;
     const int t = threadIdx.x;
@@ -251,6 +287,7 @@ __device__ __forceinline__ void sort_medium(const int *__restrict__ idx, int s, 
         if (i < n) {
             const unsigned c = (unsigned)idx[s + i];
             bad |= c >= (unsigned)colA;
+            dups |= not_ascending(ptr, idx, rows, bm, m.b, s, i, (int)c);
             x[r] = (K)(c & cmask) << 32 | (unsigned)i;
         }
     }
@@ -310,19 +347,20 @@ __global__ __launch_bounds__(kMediumThreads) void sort_medium_kernel(const int *
     __shared__ unsigned long long lds[kMedium];
     __shared__ int heads[kMediumThreads / 64];
     const int nm = min(cnt->nmedium, medium_cap);
-    bool bad = false;
+    bool bad = false, dups = false;
     for (int j = blockIdx.x; j < nm; j += gridDim.x) {
         const Big m = medium[j];
         int s, n;
         block_range(ptr, rows, nnz, bm, tilem, m.b, s, n);
         if (n > 4 * kMediumThreads)
-            sort_medium<8>(idx, s, n, cmask, colA, m, bn, words, nt, units, lds, heads, bad);
+            sort_medium<8>(ptr, idx, rows, bm, s, n, cmask, colA, m, bn, words, nt, units, lds, heads, bad, dups);
         else if (n > 2 * kMediumThreads)
-            sort_medium<4>(idx, s, n, cmask, colA, m, bn, words, nt, units, lds, heads, bad);
+            sort_medium<4>(ptr, idx, rows, bm, s, n, cmask, colA, m, bn, words, nt, units, lds, heads, bad, dups);
         else
-            sort_medium<2>(idx, s, n, cmask, colA, m, bn, words, nt, units, lds, heads, bad);
+            sort_medium<2>(ptr, idx, rows, bm, s, n, cmask, colA, m, bn, words, nt, units, lds, heads, bad, dups);
     }
     if (bad) cnt->bad = 1;
+    if (dups) cnt->dups = 1;
 }
 
 // Huge blocks: grid (blocks, kHugeY) of workgroups.
@@ -337,14 +375,16 @@ __global__ __launch_bounds__(kThreads) void huge_keys_kernel(const int *__restri
     const Big h = huge[j];
     int s, n;
     block_range(ptr, rows, nnz, bm, tilem, h.b, s, n);
-    bool bad = false;
+    bool bad = false, dups = false;
     for (long long i = blockIdx.y * kThreads + threadIdx.x; i < n; i += kHugeY * kThreads) {
         const unsigned c = (unsigned)idx[s + i];
         bad |= c >= (unsigned)colA;
+        dups |= not_ascending(ptr, idx, rows, bm, h.b, s, (int)i, (int)c);
         key[h.off + i] = (unsigned long long)j << cbits | (c & ((1ull << cbits) - 1ull));
         pos[h.off + i] = (unsigned)i;
     }
     if (bad) cnt->bad = 1;
+    if (dups) cnt->dups = 1;
 }
 
 // The sorted words of the huge blocks, and the columns each unit starts
@@ -482,12 +522,18 @@ typedef uint32_t tu4 __attribute__((ext_vector_type(4), may_alias));
 
 // Wave u < tilem: the tiles of row-block u if it has at most kSmall entries;
 // wave tilem + k: the tiles that start in unit k.  BM, BN: the class's tile
-// shape, or 0 with any shape in bm_, bn_.
-// A wave stages a window of tiles in 4 KB of LDS (one tile at least: 8 KB
-// for the widest generic shape) -- enough for 16 tiles of 256 bytes, the
-// most that two 64-entry steps of distinct columns reach -- so eight
-// workgroups of four waves fit on a CU.
-template <typename V, int BM, int BN>
+// shape, or 0 with any shape in bm_, bn_.  DUP: a slot may have several
+// entries (some row's columns do not ascend).
+// Bound by its stores when it keeps enough loads in flight: a wave reads the
+// words, then the values and columns, of kBatch x 64 entries at a time (two
+// round trips to memory per 256 entries), and stages a window of tiles in 4
+// KB of LDS (one tile at least: 8 KB for the widest generic shape), so that
+// eight workgroups of four waves fit on a CU.  RMAT scale 22, tf32 8-row
+// tiles (4.6 GB written): 2.05 ms; 3.48 ms with 64 entries a time, each
+// looking at its neighbours for duplicates.  16-row tiles of a power-law
+// matrix (1.1 GB): 0.345 ms, before 0.530.
+constexpr int kBatch = 4;
+template <typename V, int BM, int BN, bool DUP>
 __global__ __launch_bounds__(kThreads) void fill_kernel(const int *__restrict__ ptr, const int *__restrict__ idx,
                                                         const V *__restrict__ val, int rows, int nnz, int bm_, int bn_,
                                                         int tilem, const unsigned *__restrict__ words,
@@ -509,14 +555,17 @@ __global__ __launch_bounds__(kThreads) void fill_kernel(const int *__restrict__ 
     if (u == 0 && lane == 0) tile_nnz[tilenum] = nnz;
     Unit un{(int)u, 0, 0, 0};
     if (u >= tilem) un = units[u - tilem];
-    const int b = un.b;
+    const int b = __builtin_amdgcn_readfirstlane(un.b);
     int s, n;
     block_range(ptr, rows, nnz, bm, tilem, b, s, n);
+    s = __builtin_amdgcn_readfirstlane(s);
+    n = __builtin_amdgcn_readfirstlane(n);
     if (n == 0 || (u < tilem && n > kSmall)) return;
     const int t0 = tile_ptr[b], nt = tile_ptr[b + 1] - t0;
+    int q0 = __builtin_amdgcn_readfirstlane(un.p0), rk = __builtin_amdgcn_readfirstlane(un.rank0);
     // the tiles whose first column starts here
-    const int tb = (un.rank0 + bn - 1) / bn;
-    const int te = (long long)un.p0 + kSmall >= n ? nt : min(nt, (un.rank1 + bn - 1) / bn);
+    const int tb = (rk + bn - 1) / bn;
+    const int te = __builtin_amdgcn_readfirstlane((long long)q0 + kSmall >= n ? nt : min(nt, (un.rank1 + bn - 1) / bn));
     if (tb >= te) return;
     const int slots = bm * bn, mw = (slots + 63) / 64;
     const int tile_bytes = slots * (int)sizeof(V);       // a multiple of 16: bm is a multiple of 8
@@ -524,80 +573,122 @@ __global__ __launch_bounds__(kThreads) void fill_kernel(const int *__restrict__ 
     char *stage = stage_all[wid];
     unsigned long long *map = map_all[wid];
     int *rowoff = row_all[wid];
-    // first entry of each row after the first; rows past the end never match
+    // first entry of each row; rows past the end never match
+    int mine = 0x7fffffff;
     if (lane < bm) {
         const long long r = (long long)b * bm + lane;
-        rowoff[lane] = r < rows ? ptr[r] - s : 0x7fffffff;
+        if (r < rows) mine = ptr[r] - s;
+        rowoff[lane] = mine;
+    }
+    constexpr bool kScalarRows = BM == 8 || BM == 16;    // their offsets fit the scalar registers
+    int off[kScalarRows ? BM : 1];
+    if constexpr (kScalarRows) {
+#pragma unroll
+        for (int j = 0; j < BM; ++j) off[j] = __builtin_amdgcn_readlane(mine, j);
     }
     auto row_of = [&](int i) {             // the last row that starts at or before entry i
         int lo = 0;
-        for (int d = bm / 2; d >= 1; d /= 2)
-            if (rowoff[lo + d] <= i) lo += d;
+        if constexpr (kScalarRows) {
+#pragma unroll
+            for (int j = 1; j < BM; ++j) lo += i >= off[j] ? 1 : 0;
+        } else {
+            for (int d = bm / 2; d >= 1; d /= 2)
+                if (rowoff[lo + d] <= i) lo += d;
+        }
         return lo;
     };
-    int p = un.p0, rk = un.rank0;
-    for (int w0 = tb; w0 < te; w0 += wt) {
-        const int w1 = min(w0 + wt, te), nw = w1 - w0;
-        for (int k = lane; k < nw * tile_bytes / 16; k += 64) ((tu4 *)stage)[k] = tu4{0u, 0u, 0u, 0u};
-        for (int k = lane; k < nw * mw; k += 64) map[k] = 0ull;
+    int w0 = tb, w1 = min(tb + wt, te);    // the window
+    auto clear = [&]() {
+        for (int k = lane; k < (w1 - w0) * tile_bytes / 16; k += 64) ((tu4 *)stage)[k] = tu4{0u, 0u, 0u, 0u};
+        for (int k = lane; k < (w1 - w0) * mw; k += 64) map[k] = 0ull;
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        for (;;) {
-            const int q = p + lane;
-            const bool in = q < n;
-            const unsigned w = in ? words[s + q] : 0u;
-            const int i = (int)(w & ~kHead);
-            const unsigned long long hm = __ballot(in && (w & kHead));
-            const int rank = rk + __popcll(hm & (2ull << lane) - 1ull) - 1;
-            const int tile = rank >= 0 ? (int)((unsigned)rank / (unsigned)bn) : 0;
-            const bool act = in && tile < w1;
-            const unsigned long long am = __ballot(act);
-            const int row = row_of(i);
-            // the entries before and after this one in sorted order
-            unsigned wb = __shfl_up(w, 1), wa = __shfl_down(w, 1);
-            int rb = __shfl_up(row, 1), ra = __shfl_down(row, 1);
-            if (lane == 0 && q > 0) {
-                wb = words[s + q - 1];
-                rb = row_of((int)(wb & ~kHead));
-            }
-            bool more = q + 1 < n;
-            if (lane == 63 && more) {
-                wa = words[s + q + 1];
-                ra = row_of((int)(wa & ~kHead));
-            }
-            if (act && tile >= w0) {
-                const bool head = (w & kHead) != 0;
-                const int col = rank - tile * bn;
-                if (head) {
-                    colidx[(size_t)t0 * bn + rank] = idx[s + i];
-                    if (col == 0) tile_nnz[t0 + tile] = s + q;
-                }
-                if (head || rb != row) {   // the first entry of its slot
-                    V v = add_round((V)0, val[s + i]);
-                    more = more && !(wa & kHead) && ra == row;
-                    for (int k = q + 1; more;) {
-                        v = add_round(v, val[s + (int)(wa & ~kHead)]);
-                        more = ++k < n;
-                        if (more) {
-                            wa = words[s + k];
-                            more = !(wa & kHead) && row_of((int)(wa & ~kHead)) == row;
-                        }
-                    }
-                    const int slot = row * bn + col, tl = tile - w0;
-                    ((V *)stage)[tl * slots + slot] = v;
-                    atomicOr((unsigned *)map + 2 * (tl * mw) + slot / 32, 1u << (slot & 31));
-                }
-            }
-            const int na = __popcll(am);
-            p += na;
-            rk += __popcll(hm & am);
-            if (na < 64) break;
-        }
+    };
+    auto flush = [&]() {
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         tu4 *out = (tu4 *)((char *)dense + (size_t)(t0 + w0) * tile_bytes);
-        for (int k = lane; k < nw * tile_bytes / 16; k += 64) out[k] = ((const tu4 *)stage)[k];
-        for (int k = lane; k < nw * mw; k += 64) bitmap[(size_t)(t0 + w0) * mw + k] = map[k];
+        for (int k = lane; k < (w1 - w0) * tile_bytes / 16; k += 64)
+            __builtin_nontemporal_store(((const tu4 *)stage)[k], out + k);
+        for (int k = lane; k < (w1 - w0) * mw; k += 64) bitmap[(size_t)(t0 + w0) * mw + k] = map[k];
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    };
+    clear();
+    int prow = -1;                         // row of the entry before this batch
+    if (DUP && q0 > 0) prow = row_of((int)(words[s + q0 - 1] & ~kHead));
+    for (; q0 < n && w0 < te; q0 += 64 * kBatch) {
+        unsigned w[kBatch];
+        int rank[kBatch], c[kBatch];
+        V v[kBatch];
+#pragma unroll
+        for (int k = 0; k < kBatch; ++k) {
+            const int q = q0 + 64 * k + lane;
+            w[k] = q < n ? words[s + q] : 0u;
+        }
+#pragma unroll
+        for (int k = 0; k < kBatch; ++k) {
+            const int q = q0 + 64 * k + lane, i = (int)(w[k] & ~kHead);
+            v[k] = q < n ? val[s + i] : (V)0;
+            c[k] = (w[k] & kHead) ? idx[s + i] : 0;
+        }
+#pragma unroll
+        for (int k = 0; k < kBatch; ++k) {
+            const unsigned long long hm = __ballot((w[k] & kHead) != 0);
+            rank[k] = rk + __popcll(hm & ((2ull << lane) - 1ull)) - 1;
+            rk += __popcll(hm);
+        }
+        bool skip[kBatch];                 // not the first entry of its slot
+        if constexpr (DUP) {
+#pragma unroll
+            for (int k = 0; k < kBatch; ++k) {
+                const int q = q0 + 64 * k + lane, row = row_of((int)(w[k] & ~kHead));
+                int before = __shfl_up(row, 1);
+                if (lane == 0) before = prow;
+                skip[k] = !(w[k] & kHead) && before == row;
+                prow = __builtin_amdgcn_readlane(row, 63);
+                // the first entry of a slot adds up the ones that follow
+                if (q < n && !skip[k]) {
+                    v[k] = add_round((V)0, v[k]);
+                    for (int j = q + 1; j < n; ++j) {
+                        const unsigned wa = words[s + j];
+                        if ((wa & kHead) || row_of((int)wa) != row) break;
+                        v[k] = add_round(v[k], val[s + (int)wa]);
+                    }
+                }
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < kBatch; ++k) {
+                skip[k] = false;
+                v[k] = add_round((V)0, v[k]);
+            }
+        }
+        const int last = (rk - 1) / bn;    // the last tile reached
+        for (;;) {
+#pragma unroll
+            for (int k = 0; k < kBatch; ++k) {
+                const int q = q0 + 64 * k + lane, i = (int)(w[k] & ~kHead);
+                const int tile = (int)((unsigned)max(rank[k], 0) / (unsigned)bn);
+                if (q < n && tile >= w0 && tile < w1) {
+                    const int col = rank[k] - tile * bn, tl = tile - w0;
+                    if (w[k] & kHead) {
+                        colidx[(size_t)t0 * bn + rank[k]] = c[k];
+                        if (col == 0) tile_nnz[t0 + tile] = s + q;
+                    }
+                    if (!skip[k]) {
+                        const int slot = row_of(i) * bn + col;
+                        ((V *)stage)[tl * slots + slot] = v[k];
+                        atomicOr((unsigned *)map + 2 * (tl * mw) + ((unsigned)slot >> 5), 1u << (slot & 31));
+                    }
+                }
+            }
+            if (last < w1) break;
+            flush();
+            w0 = w1;
+            if (w0 >= te) break;
+            w1 = min(w0 + wt, te);
+            clear();
+        }
     }
+    if (w0 < te) flush();
     if (te == nt) {
         // the block's last tile repeats its last column
         const int last = idx[s + (int)(words[s + n - 1] & ~kHead)];
@@ -912,19 +1003,24 @@ int tile_create_device(tsp_dev_tiles *out, int rows, int colA, long long nnz, co
                                                 (std::remove_const_t<std::remove_pointer_t<decltype(v)>> *)out->d_val,
                                                 (unsigned long long *)out->d_bitmap);
     };
-    if (prec == TSP_PREC_FP16) {
-        const _Float16 *v = (const _Float16 *)d_val;
-        if (BM == 8 && BN == 16) fill(fill_kernel<_Float16, 8, 16>, v);
-        else if (BM == 16 && BN == 16) fill(fill_kernel<_Float16, 16, 16>, v);
-        else if (BM == 64 && BN == 32) fill(fill_kernel<_Float16, 64, 32>, v);
-        else fill(fill_kernel<_Float16, 0, 0>, v);
-    } else {
-        const float *v = (const float *)d_val;
-        if (BM == 8 && BN == 8) fill(fill_kernel<float, 8, 8>, v);
-        else if (BM == 16 && BN == 8) fill(fill_kernel<float, 16, 8>, v);
-        else if (BM == 64 && BN == 16) fill(fill_kernel<float, 64, 16>, v);
-        else fill(fill_kernel<float, 0, 0>, v);
-    }
+    const auto shape = [&](auto dup) {
+        constexpr bool DUP = decltype(dup)::value;
+        if (prec == TSP_PREC_FP16) {
+            const _Float16 *v = (const _Float16 *)d_val;
+            if (BM == 8 && BN == 16) fill(fill_kernel<_Float16, 8, 16, DUP>, v);
+            else if (BM == 16 && BN == 16) fill(fill_kernel<_Float16, 16, 16, DUP>, v);
+            else if (BM == 64 && BN == 32) fill(fill_kernel<_Float16, 64, 32, DUP>, v);
+            else fill(fill_kernel<_Float16, 0, 0, DUP>, v);
+        } else {
+            const float *v = (const float *)d_val;
+            if (BM == 8 && BN == 8) fill(fill_kernel<float, 8, 8, DUP>, v);
+            else if (BM == 16 && BN == 8) fill(fill_kernel<float, 16, 8, DUP>, v);
+            else if (BM == 64 && BN == 16) fill(fill_kernel<float, 64, 16, DUP>, v);
+            else fill(fill_kernel<float, 0, 0, DUP>, v);
+        }
+    };
+    if (h.dups) shape(std::true_type{});
+    else shape(std::false_type{});
     TCHK(hipGetLastError());
     return (int)hipStreamSynchronize(s);
 }
