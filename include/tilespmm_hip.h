@@ -358,6 +358,12 @@ int tsp_gather_kernel(const void *table, size_t table_bytes, int row_bytes, int 
 int tsp_gather_index_stream(const void *d_table, long long table_rows, int row_bytes, const int *d_idx, long long n,
                             void *d_sink, void *stream);
 
+/* Zeroes rows 8 u .. 8 u + 7 (below c_rows) of C [c_rows][colB_p] for the n
+ * entries u of d_units, asynchronously on `stream`: the part of C that the
+ * launches of a step add to (split row-blocks) or leave alone.  colB_p is a
+ * multiple of 4. */
+int tsp_zero_rows(float *d_C, int c_rows, int colB_p, const int *d_units, int n, void *stream);
+
 /* ---- Hot B rows ------------------------------------------------------------
  * B is allocated with spare rows after row colA; hot slot s is row colA + s
  * and holds a copy of B row hot[s].  A tile column index colA + s then reads

@@ -427,6 +427,12 @@ __global__ __launch_bounds__(256) void split_bf16_kernel(const uint32_t *__restr
 }
 }  // namespace tsp
 
+int tsp_zero_rows(float *d_C, int c_rows, int colB_p, const int *d_units, int n, void *stream)
+{
+    if (c_rows < 0 || colB_p <= 0 || colB_p % 4 || n < 0 || (n > 0 && (!d_C || !d_units))) return TSP_EINVAL;
+    return tsp::launch_zero_rows(d_C, c_rows, colB_p, d_units, n, (hipStream_t)stream);
+}
+
 int tsp_split_bf16_device(const void *d_src, void *d_dst, size_t n, void *stream)
 {
     if (n && (!d_src || !d_dst)) return TSP_EINVAL;

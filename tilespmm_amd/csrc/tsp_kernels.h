@@ -145,6 +145,7 @@ int launch(int bm, int prec, int ntasks, int colB_p, const void *val, const uint
            int placement = kPlaceContiguous, bool lane_idx = false, int b_rows = 0, int panel_rows = 0,
            int panel_lag = 1, int *sync = nullptr, long long sync_ints = 0, bool sync_reset = false,
            bool pair = false, int opts = 0);
+int launch_zero_rows(float *C, int c_rows, int colB_p, const int *units, int n, hipStream_t s);
 int launch_copy(void *dst, const void *src, size_t bytes, hipStream_t s);
 constexpr int kGatherBlocks = 8192;      // gather probe grid: 8192 x 256 threads
 int launch_gather(const void *table, size_t table_bytes, int row_bytes, int iters, unsigned seed, void *sink,

@@ -33,6 +33,28 @@ __global__ __launch_bounds__(256) void fill_kernel(int *__restrict__ p, long lon
         p[i] = 0;
 }
 
+// Rows 8 u .. 8 u + 7 of C for the listed units u, 16 bytes per thread and
+// step.  Bound by its stores.
+__global__ __launch_bounds__(256) void zero_rows_kernel(u4 *__restrict__ C, int c_rows, int row_vecs,
+                                                        const int *__restrict__ units, int n)
+{
+    const long long total = (long long)n * 8 * row_vecs;
+    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < total;
+         i += (long long)gridDim.x * blockDim.x) {
+        const long long row = i / row_vecs;                // of the list
+        const long long r = (long long)units[row >> 3] * 8 + (row & 7);
+        if (r < c_rows) C[r * row_vecs + (i - row * row_vecs)] = u4{0u, 0u, 0u, 0u};
+    }
+}
+
+int launch_zero_rows(float *C, int c_rows, int colB_p, const int *units, int n, hipStream_t s)
+{
+    if (n <= 0) return 0;
+    const long long blocks = ((long long)n * 2 * colB_p + 255) / 256;
+    zero_rows_kernel<<<(unsigned)std::min<long long>(blocks, 65536), 256, 0, s>>>((u4 *)C, c_rows, colB_p / 4, units, n);
+    return (int)hipGetLastError();
+}
+
 // ---------------------------------------------------------------------------
 // Dispatch.
 // ---------------------------------------------------------------------------
