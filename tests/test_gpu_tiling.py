@@ -226,3 +226,40 @@ def test_device_tiles_other_widths(gpu, orc, prec, bm, bn):
     say(f"device tiles {bm}x{bn} prec={prec}")
     d = gpu.tile_create_device(sub, cols, bm, prec, bn)
     assert_same(d, orc.tile_create(rows, cols, rp, ci, bits, prec, bm, bn), prec, f"{bm}x{bn}")
+
+
+# Blocks past the wave's size whose rows ascend are merged instead of sorted:
+# rows of very different lengths (all entries in one row, empty rows first
+# and last), runs whose columns do not overlap, and one block each way beside
+# one with a duplicate.
+@pytest.mark.parametrize("entries", [1025, 2047, 4096, 4097, 8192, 8193, 12289, 70001])
+@pytest.mark.parametrize("prec,bm", [(0, 8), (0, 16), (1, 64)])
+@pytest.mark.parametrize("shape", ["even", "one row", "skewed", "apart"])
+def test_device_tiles_ascending_rows(gpu, orc, entries, prec, bm, shape):
+    rng = np.random.default_rng(entries + bm)
+    cols = 80021
+    if shape == "one row":
+        part = np.zeros(bm, np.int64)
+        part[int(rng.integers(bm))] = entries
+    elif shape == "skewed":
+        part = rng.multinomial(entries, rng.dirichlet(np.ones(bm) * 0.2))
+    else:
+        part = np.full(bm, entries // bm, np.int64)
+        part[0] += entries - part.sum()
+    rows_ci = []
+    for r, k in enumerate(part):
+        if shape == "apart":                        # row r's columns all before row r + 1's
+            lo, hi = cols * r // bm, cols * (r + 1) // bm
+            rows_ci.append(np.sort(rng.choice(np.arange(lo, hi), min(int(k), hi - lo), replace=False)))
+        else:
+            rows_ci.append(np.sort(rng.choice(cols, int(k), replace=False)))
+    few = [np.sort(rng.choice(cols, int(rng.integers(0, 6)), replace=False)) for _ in range(bm + 3)]
+    for dup in (False, True):
+        all_rows = few[:bm] + rows_ci + rows_ci[::-1] + few[bm:]
+        if dup:
+            j = bm + int(np.argmax([len(c) for c in rows_ci]))
+            all_rows[j] = np.concatenate([all_rows[j], all_rows[j][-1:]])
+        rp = np.concatenate([[0], np.cumsum([len(c) for c in all_rows])]).astype(np.int32)
+        ci = np.concatenate(all_rows).astype(np.int32)
+        store, bits = values_for(rng, len(ci), prec)
+        check_vs_oracle(gpu, orc, len(all_rows), cols, rp, ci, prec, bm, store, bits, f"{entries} {shape} dup={dup}")

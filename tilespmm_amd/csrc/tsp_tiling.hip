@@ -3,12 +3,15 @@
 // conversion (tilespmm_amd/host/tiles.cpp).
 //
 //   1. Each row-block's entries are sorted by (column, position) where they
-//      lie: a block of up to kSmall entries by one wave in registers, up to
-//      kMedium by one workgroup through LDS, larger ones (a dense row of a
-//      circuit, the hubs of a power-law graph) by one rocPRIM radix sort over
-//      the entries of all such blocks.  The only scratch is one word per
-//      entry: its position inside the block, bit 31 set where a new column
-//      starts.  Entries of one (block, column) pair keep the CSR order.
+//      lie: a block of up to kSmall entries by one wave in registers.  A
+//      larger one whose rows ascend, as nearly all do, is its rows merged
+//      pairwise: up to kMedium entries by one workgroup through LDS, beyond
+//      (a dense row of a circuit, the hubs of a power-law graph) by many
+//      through memory.  Rows in another order are sorted by the workgroup or
+//      by a rocPRIM radix sort.  The only scratch is one word per entry
+//      (16 bytes for the largest blocks): its position inside the block, bit
+//      31 set where a new column starts.  Entries of one (block, column) pair
+//      keep the CSR order.
 //   2. ceil(distinct / BN) tiles per block; one chained scan -> tile_ptr.
 //   3. One wave per block (per kSmall sorted entries of a larger block) walks
 //      its sorted entries, builds its tiles a few at a time in LDS -- values,
@@ -22,7 +25,7 @@
 //
 // The conversion is bound by memory traffic: it reads the column indices
 // twice, the values once, the 4-byte scratch twice, and writes the tiles
-// once.  RMAT scale 22 (128M entries) to tf32 8-row tiles: 7.5 ms of kernels,
+// once.  RMAT scale 22 (128M entries) to tf32 8-row tiles: 4.6 ms of kernels,
 // against 28 ms for a global radix sort of 8-byte keys over all entries with
 // cleared output arrays filled by one thread per column run.
 #include <cstring>
@@ -33,6 +36,7 @@
 
 #include <mutex>
 #include <type_traits>
+#include <utility>
 
 #include "../../include/tilespmm_hip.h"
 #include "tsp_kernels.h"
@@ -85,7 +89,9 @@ struct Counters {
     long long total;                       // tiles
     int bad;                               // a column outside [0, colA), or row pointers out of order
     int dups;                              // some row's columns do not ascend: a slot may have several entries
-    int nunits, nmedium;
+    int odd;                               // ... in a globally sorted block
+    int nunits;
+    int nmerge[2], nsort;                  // blocks of up to kMedium / 2 and kMedium entries; those to sort after all
     int ticket;                            // of the chained scan
 };
 
@@ -228,9 +234,9 @@ __global__ __launch_bounds__(kThreads) void sort_blocks_kernel(const int *__rest
             const int u = atomicAdd(&cnt->nunits, ns);
             bad = u < 0 || u > unit_cap - ns;    // only row pointers out of order get there
             if (!bad && n <= kMedium) {
-                const int j = atomicAdd(&cnt->nmedium, 1);
+                const int k = n > kMedium / 2 ? 1 : 0, j = atomicAdd(&cnt->nmerge[k], 1);
                 bad = j < 0 || j >= medium_cap;
-                if (!bad) medium[j] = Big{b, u, 0};
+                if (!bad) medium[(size_t)k * medium_cap + j] = Big{b, u, 0};
             } else if (!bad) {
                 const unsigned long long at = atomicAdd(&cnt->huge, (1ull << 40) + (unsigned long long)n);
                 const long long j = (long long)(at >> 40);
@@ -269,13 +275,174 @@ __device__ __forceinline__ bool not_ascending(const int *__restrict__ ptr, const
     return true;
 }
 
-// Sorts one block of at most kMediumThreads * R entries by the workgroup.
+// ---- merging the rows of a block ---------------------------------------------
+// A block whose rows ascend is its bm rows merged pairwise in log2(bm)
+// rounds.  Keys are column << 32 | position, all different.  A thread writes
+// kMergePer outputs of a round: a binary search along its diagonal of the
+// two runs finds where it starts (merge path), then it takes the smaller
+// head.  In LDS, element i lies at i + i / kMergePer, so that the threads'
+// consecutive outputs fall in different banks.  RMAT scale 22, 8-row blocks:
+// 0.61 ms for the medium blocks (31M entries), 1.25 ms for the huge ones
+// (46M); sorting networks of the whole workgroup took 3.0 ms (mostly lane
+// exchanges), a radix sort of 12-byte pairs 1.75 ms.
+constexpr int kMergePer = 8;
+__device__ __forceinline__ int lds_at(int i) { return i + i / kMergePer; }
+
+// How many of the first k outputs come from the first of two runs in LDS
+// (la keys from a, lb keys from b).
+__device__ __forceinline__ int diagonal(const unsigned long long *lds, int a, int la, int b, int lb, int k)
+{
+    int lo = max(0, k - lb), hi = min(k, la);
+    while (lo < hi) {
+        const int mid = (lo + hi) / 2;
+        if (lds[lds_at(a + mid)] < lds[lds_at(b + k - 1 - mid)]) lo = mid + 1;
+        else hi = mid;
+    }
+    return lo;
+}
+
+// Outputs o .. o + kMergePer - 1 (below n) of merging runs 2gj .. 2gj + g - 1
+// with runs 2gj + g .. 2gj + 2g - 1 for every j; run r is off[r] .. off[r + 1].
+__device__ __forceinline__ void merge_round(const unsigned long long *lds, const int *off, int bm, int g, int n, int o,
+                                            unsigned long long (&y)[kMergePer])
+{
+    if (o >= n) return;
+    int lo = 0, hi = bm / (2 * g) - 1;                 // the last pair that starts at or before o
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) / 2;
+        if (off[2 * g * mid] <= o) lo = mid;
+        else hi = mid - 1;
+    }
+    int j = lo;
+    int a = off[2 * g * j], ae = off[2 * g * j + g], b = ae, be = off[2 * g * (j + 1)];
+    const int d = diagonal(lds, a, ae - a, b, be - b, o - a);
+    b += o - a - d;
+    a += d;
+    unsigned long long ka = a < ae ? lds[lds_at(a)] : ~0ull, kb = b < be ? lds[lds_at(b)] : ~0ull;
+#pragma unroll
+    for (int e = 0; e < kMergePer; ++e) {
+        if (o + e >= n) break;
+        while (a == ae && b == be) {                   // (pairs cover all n positions)
+            ++j;
+            a = off[2 * g * j];
+            b = ae = off[2 * g * j + g];
+            be = off[2 * g * (j + 1)];
+            ka = a < ae ? lds[lds_at(a)] : ~0ull;
+            kb = b < be ? lds[lds_at(b)] : ~0ull;
+        }
+        if (ka < kb) {
+            y[e] = ka;
+            ++a;
+            ka = a < ae ? lds[lds_at(a)] : ~0ull;
+        } else {
+            y[e] = kb;
+            ++b;
+            kb = b < be ? lds[lds_at(b)] : ~0ull;
+        }
+    }
+}
+
+// Workgroups share out the listed blocks, of at most THREADS * kMergePer
+// entries.  One whose rows do not ascend goes on the list for
+// sort_medium_kernel.
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void merge_medium_kernel(const int *__restrict__ ptr, const int *__restrict__ idx,
+                                                               int rows, int nnz, int bm, int bn, int tilem,
+                                                               unsigned cmask, int colA, unsigned *__restrict__ words,
+                                                               int *__restrict__ nt, const Big *__restrict__ list,
+                                                               const int *__restrict__ nlist, int cap,
+                                                               Big *__restrict__ unsorted, Unit *__restrict__ units,
+                                                               Counters *__restrict__ cnt)
+{
+    constexpr int N = THREADS * kMergePer;
+    __shared__ unsigned long long lds[N + N / kMergePer];
+    __shared__ int off[65];
+    __shared__ int heads[THREADS / 64];
+    const int t = threadIdx.x;
+    const int nl = min(*nlist, cap);
+    bool bad = false;
+    for (int l = blockIdx.x; l < nl; l += gridDim.x) {
+        const Big m = list[l];
+        int s, n;
+        block_range(ptr, rows, nnz, bm, tilem, m.b, s, n);
+        n = min(n, N);
+        if (t <= bm) {
+            const long long r = (long long)m.b * bm + t;
+            off[t] = t == 0 ? 0 : t == bm || r >= rows ? n : min(max(ptr[r] - s, 0), n);
+        }
+#pragma unroll
+        for (int r = 0; r < kMergePer; ++r) {
+            const int i = r * THREADS + t;
+            if (i < n) {
+                const unsigned c = (unsigned)idx[s + i];
+                bad |= c >= (unsigned)colA;
+                lds[lds_at(i)] = (unsigned long long)(c & cmask) << 32 | (unsigned)i;
+            }
+        }
+        __syncthreads();
+        bool odd = t < bm && off[t + 1] < off[t];
+#pragma unroll
+        for (int r = 0; r < kMergePer; ++r) {
+            const int i = r * THREADS + t;
+            if (i > 0 && i < n && (lds[lds_at(i)] >> 32) <= (lds[lds_at(i - 1)] >> 32)) {
+                bool start = false;
+                for (int k = 1; k < bm; ++k) start |= off[k] == i;
+                odd |= !start;
+            }
+        }
+        if (__syncthreads_or(odd)) {
+            if (t == 0) {
+                cnt->dups = 1;
+                unsorted[atomicAdd(&cnt->nsort, 1)] = m;   // each listed block once: within both lists' room
+            }
+            __syncthreads();
+            continue;
+        }
+        const int o = t * kMergePer;
+        unsigned long long y[kMergePer];
+        for (int g = 1; g < bm; g *= 2) {
+            merge_round(lds, off, bm, g, n, o, y);
+            __syncthreads();
+#pragma unroll
+            for (int e = 0; e < kMergePer; ++e)
+                if (o + e < n) lds[lds_at(o + e)] = y[e];
+            __syncthreads();
+        }
+        unsigned before = o > 0 && o < n ? (unsigned)(lds[lds_at(o - 1)] >> 32) : 0u;
+        int mine = 0;
+#pragma unroll
+        for (int e = 0; e < kMergePer; ++e) {
+            const bool in = o + e < n;
+            const bool head = in && (o + e == 0 || (unsigned)(y[e] >> 32) != before);
+            before = (unsigned)(y[e] >> 32);
+            mine += __popcll(__ballot(head));
+            if (in) words[s + o + e] = (unsigned)y[e] | (head ? kHead : 0u);
+        }
+        // a wave holds 64 kMergePer sorted entries
+        if ((t & 63) == 0) heads[t >> 6] = mine;
+        __syncthreads();
+        if (t == 0) {
+            constexpr int PW = kSmall / (64 * kMergePer);
+            int run = 0;
+            for (int u = 0; u * kSmall < n; ++u) {
+                int k = 0;
+                for (int w = 0; w < PW; ++w) k += heads[u * PW + w];
+                units[m.unit0 + u] = Unit{m.b, u * kSmall, run, run + k};
+                run += k;
+            }
+            nt[m.b] = (run + bn - 1) / bn;
+        }
+        __syncthreads();
+    }
+    if (bad) cnt->bad = 1;
+}
+
+// Sorts one block of at most kMediumThreads * R entries by the workgroup,
+// whatever the order of its rows' columns.
 template <int R>
-__device__ __forceinline__ void sort_medium(const int *__restrict__ ptr, const int *__restrict__ idx, int rows, int bm,
-                                            int s, int n, unsigned cmask, int colA, Big m, int bn,
+__device__ __forceinline__ void sort_medium(const int *__restrict__ idx, int s, int n, unsigned cmask, Big m, int bn,
                                             unsigned *__restrict__ words, int *__restrict__ nt,
-                                            Unit *__restrict__ units, unsigned long long *lds, int *heads, bool &bad,
-                                            bool &dups)
+                                            Unit *__restrict__ units, unsigned long long *lds, int *heads)
 {
     typedef unsigned long long K;
     const int t = threadIdx.x;
@@ -285,10 +452,7 @@ __device__ __forceinline__ void sort_medium(const int *__restrict__ ptr, const i
         const int i = r * kMediumThreads + t;
         x[r] = ~0ull;
         if (i < n) {
-            const unsigned c = (unsigned)idx[s + i];
-            bad |= c >= (unsigned)colA;
-            dups |= not_ascending(ptr, idx, rows, bm, m.b, s, i, (int)c);
-            x[r] = (K)(c & cmask) << 32 | (unsigned)i;
+            x[r] = (K)((unsigned)idx[s + i] & cmask) << 32 | (unsigned)i;
         }
     }
     bitonic<2, kMediumThreads * R>(x, t, [&](const K (&v)[R], K (&y)[R], int d, bool flip) {
@@ -334,37 +498,35 @@ __device__ __forceinline__ void sort_medium(const int *__restrict__ ptr, const i
     __syncthreads();
 }
 
-// Workgroups share out the medium blocks.
+// Workgroups share out the blocks of the list.
 __global__ __launch_bounds__(kMediumThreads) void sort_medium_kernel(const int *__restrict__ ptr,
                                                                      const int *__restrict__ idx, int rows, int nnz,
                                                                      int bm, int bn, int tilem, unsigned cmask,
-                                                                     int colA, unsigned *__restrict__ words,
+                                                                     unsigned *__restrict__ words,
                                                                      int *__restrict__ nt,
-                                                                     const Big *__restrict__ medium, int medium_cap,
+                                                                     const Big *__restrict__ list, int cap,
                                                                      Unit *__restrict__ units,
-                                                                     Counters *__restrict__ cnt)
+                                                                     const Counters *__restrict__ cnt)
 {
     __shared__ unsigned long long lds[kMedium];
     __shared__ int heads[kMediumThreads / 64];
-    const int nm = min(cnt->nmedium, medium_cap);
-    bool bad = false, dups = false;
-    for (int j = blockIdx.x; j < nm; j += gridDim.x) {
-        const Big m = medium[j];
+    const int nl = min(cnt->nsort, cap);
+    for (int j = blockIdx.x; j < nl; j += gridDim.x) {
+        const Big m = list[j];
         int s, n;
         block_range(ptr, rows, nnz, bm, tilem, m.b, s, n);
-        if (n > 4 * kMediumThreads)
-            sort_medium<8>(ptr, idx, rows, bm, s, n, cmask, colA, m, bn, words, nt, units, lds, heads, bad, dups);
-        else if (n > 2 * kMediumThreads)
-            sort_medium<4>(ptr, idx, rows, bm, s, n, cmask, colA, m, bn, words, nt, units, lds, heads, bad, dups);
-        else
-            sort_medium<2>(ptr, idx, rows, bm, s, n, cmask, colA, m, bn, words, nt, units, lds, heads, bad, dups);
+        n = min(n, kMedium);
+        if (n > 4 * kMediumThreads) sort_medium<8>(idx, s, n, cmask, m, bn, words, nt, units, lds, heads);
+        else if (n > 2 * kMediumThreads) sort_medium<4>(idx, s, n, cmask, m, bn, words, nt, units, lds, heads);
+        else sort_medium<2>(idx, s, n, cmask, m, bn, words, nt, units, lds, heads);
     }
-    if (bad) cnt->bad = 1;
-    if (dups) cnt->dups = 1;
 }
 
-// Huge blocks: grid (blocks, kHugeY) of workgroups.
+// Huge blocks: grid (blocks, kHugeY) of workgroups.  MERGE: keys column << 32
+// | position for the merge rounds, else block << cbits | column with the
+// position apart for the radix sort.
 constexpr int kHugeY = 64;
+template <bool MERGE>
 __global__ __launch_bounds__(kThreads) void huge_keys_kernel(const int *__restrict__ ptr, const int *__restrict__ idx,
                                                              int rows, int nnz, int bm, int tilem, int cbits, int colA,
                                                              const Big *__restrict__ huge,
@@ -375,26 +537,130 @@ __global__ __launch_bounds__(kThreads) void huge_keys_kernel(const int *__restri
     const Big h = huge[j];
     int s, n;
     block_range(ptr, rows, nnz, bm, tilem, h.b, s, n);
-    bool bad = false, dups = false;
+    bool bad = false, odd = false;
+    const unsigned long long mask = (1ull << cbits) - 1ull;
     for (long long i = blockIdx.y * kThreads + threadIdx.x; i < n; i += kHugeY * kThreads) {
         const unsigned c = (unsigned)idx[s + i];
         bad |= c >= (unsigned)colA;
-        dups |= not_ascending(ptr, idx, rows, bm, h.b, s, (int)i, (int)c);
-        key[h.off + i] = (unsigned long long)j << cbits | (c & ((1ull << cbits) - 1ull));
-        pos[h.off + i] = (unsigned)i;
+        if constexpr (MERGE) {
+            odd |= not_ascending(ptr, idx, rows, bm, h.b, s, (int)i, (int)c);
+            key[h.off + i] = (c & mask) << 32 | (unsigned)i;
+        } else {
+            key[h.off + i] = (unsigned long long)j << cbits | (c & mask);
+            pos[h.off + i] = (unsigned)i;
+        }
+    }
+    if (MERGE && blockIdx.y == 0 && (int)threadIdx.x < bm) {
+        // rows in order, too
+        const long long r = (long long)h.b * bm + threadIdx.x;
+        if (r > 0 && r < rows) odd |= ptr[r] < ptr[r - 1];
     }
     if (bad) cnt->bad = 1;
-    if (dups) cnt->dups = 1;
+    if (odd) cnt->odd = 1;
+}
+
+// How many of the first k outputs come from the first of two runs (la keys at
+// A, lb at B), by a wave: 64 probes a step.
+__device__ __forceinline__ int diagonal_wave(const unsigned long long *__restrict__ A, int la,
+                                             const unsigned long long *__restrict__ B, int lb, int k, int lane)
+{
+    int lo = max(0, k - lb), hi = min(k, la);
+    while (lo < hi) {
+        const int step = (int)(((long long)hi - lo + 63) / 64);
+        const long long mid = lo + (long long)lane * step;
+        const bool less = mid < hi && A[mid] < B[k - 1 - mid];
+        const int c = __popcll(__ballot(less));            // the first c probes
+        if (c == 0) {
+            hi = lo;
+        } else {
+            const int at = lo;
+            lo = at + (c - 1) * step + 1;
+            hi = (int)min((long long)hi, at + (long long)c * step);
+        }
+    }
+    return lo;
+}
+
+// One round of merging the rows of the huge blocks, in to out: a workgroup
+// merges kMergeTile outputs of one pair through LDS at a time.
+constexpr int kMergeTile = kThreads * kMergePer;
+__global__ __launch_bounds__(kThreads) void huge_merge_kernel(const int *__restrict__ ptr, int rows, int nnz, int bm,
+                                                              int tilem, int g, const Big *__restrict__ huge,
+                                                              const unsigned long long *__restrict__ in,
+                                                              unsigned long long *__restrict__ out,
+                                                              const Counters *__restrict__ cnt)
+{
+    __shared__ unsigned long long lds[kMergeTile + kMergeTile / kMergePer];
+    __shared__ int off[65];
+    __shared__ int split[2];
+    if (cnt->odd) return;                                  // the radix sort follows
+    const Big h = huge[blockIdx.x];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    int s, n;
+    block_range(ptr, rows, nnz, bm, tilem, h.b, s, n);
+    if (t <= bm) {
+        const long long r = (long long)h.b * bm + t;
+        off[t] = t == 0 ? 0 : t == bm || r >= rows ? n : min(max(ptr[r] - s, 0), n);
+    }
+    __syncthreads();
+    int j = 0, first = 0;                                  // pair, and its first tile
+    for (int tile = blockIdx.y;; tile += kHugeY) {
+        int p = 0, m = 0, e = 0;
+        for (; j < bm / (2 * g); ++j) {
+            p = off[2 * g * j];
+            m = off[2 * g * j + g];
+            e = off[2 * g * (j + 1)];
+            const int tiles = (int)(((long long)e - p + kMergeTile - 1) / kMergeTile);
+            if (tile < first + tiles) break;
+            first += tiles;
+        }
+        if (j >= bm / (2 * g)) return;
+        const int k0 = (tile - first) * kMergeTile, k1 = (int)min((long long)k0 + kMergeTile, (long long)e - p);
+        const unsigned long long *A = in + h.off + p, *B = in + h.off + m;
+        if (wave < 2) {
+            const int d = diagonal_wave(A, m - p, B, e - m, wave ? k1 : k0, lane);
+            if (lane == 0) split[wave] = d;
+        }
+        __syncthreads();
+        const int a0 = split[0], na = split[1] - a0, nb = k1 - k0 - na;
+        for (int i = t; i < na; i += kThreads) lds[lds_at(i)] = A[a0 + i];
+        for (int i = t; i < nb; i += kThreads) lds[lds_at(na + i)] = B[k0 - a0 + i];
+        __syncthreads();
+        const int o = t * kMergePer;
+        if (o < na + nb) {
+            int a = diagonal(lds, 0, na, na, nb, o), b = na + o - a;
+            unsigned long long ka = a < na ? lds[lds_at(a)] : ~0ull, kb = b < na + nb ? lds[lds_at(b)] : ~0ull;
+            unsigned long long *y = out + h.off + p + k0 + o;
+#pragma unroll
+            for (int x = 0; x < kMergePer; ++x) {
+                if (o + x >= na + nb) break;
+                if (ka < kb) {
+                    y[x] = ka;
+                    ++a;
+                    ka = a < na ? lds[lds_at(a)] : ~0ull;
+                } else {
+                    y[x] = kb;
+                    ++b;
+                    kb = b < na + nb ? lds[lds_at(b)] : ~0ull;
+                }
+            }
+        }
+        __syncthreads();
+    }
 }
 
 // The sorted words of the huge blocks, and the columns each unit starts
 // (rank1; the ranks follow).
+template <bool MERGE>
 __global__ __launch_bounds__(kThreads) void huge_words_kernel(const int *__restrict__ ptr, int rows, int nnz, int bm,
                                                               int tilem, const Big *__restrict__ huge,
                                                               const unsigned long long *__restrict__ key,
                                                               const unsigned *__restrict__ pos,
-                                                              unsigned *__restrict__ words, Unit *__restrict__ units)
+                                                              unsigned *__restrict__ words, Unit *__restrict__ units,
+                                                              const Counters *__restrict__ cnt)
 {
+    if (MERGE && cnt->odd) return;
+    constexpr int kShift = MERGE ? 32 : 0;
     const Big h = huge[blockIdx.x];
     const int lane = threadIdx.x & 63, wave = blockIdx.y * (kThreads / 64) + (threadIdx.x >> 6);
     int s, n;
@@ -404,8 +670,9 @@ __global__ __launch_bounds__(kThreads) void huge_words_kernel(const int *__restr
         for (int i = 0; i < kSmall; i += 64) {
             const long long p = u * kSmall + i + lane;
             const bool in = p < n;
-            const bool head = in && (p == 0 || key[h.off + p] != key[h.off + p - 1]);
-            if (in) words[s + p] = pos[h.off + p] | (head ? kHead : 0u);
+            const unsigned long long x = in ? key[h.off + p] : 0ull;
+            const bool head = in && (p == 0 || x >> kShift != key[h.off + p - 1] >> kShift);
+            if (in) words[s + p] = (MERGE ? (unsigned)x : pos[h.off + p]) | (head ? kHead : 0u);
             k += __popcll(__ballot(head));
         }
         if (lane == 0) units[h.unit0 + u] = Unit{h.b, (int)(u * kSmall), 0, k};
@@ -415,8 +682,10 @@ __global__ __launch_bounds__(kThreads) void huge_words_kernel(const int *__restr
 // One workgroup per huge block: ranks of its units, its tiles.
 __global__ __launch_bounds__(kThreads) void huge_ranks_kernel(const int *__restrict__ ptr, int rows, int nnz, int bm,
                                                               int bn, int tilem, const Big *__restrict__ huge,
-                                                              Unit *__restrict__ units, int *__restrict__ nt)
+                                                              Unit *__restrict__ units, int *__restrict__ nt,
+                                                              const Counters *__restrict__ cnt, bool merged)
 {
+    if (merged && cnt->odd) return;
     using BS = rocprim::block_scan<int, kThreads>;
     __shared__ typename BS::storage_type st;
     const Big h = huge[blockIdx.x];
@@ -958,8 +1227,32 @@ int launch_scan(F in, int n, int *out, unsigned long long *state, int *ticket, l
     return (int)hipGetLastError();
 }
 
-// Sorts the entries of the `nh` huge blocks (`entries` in all) and completes
-// their words, units and tile counts.
+// Merges the rows of the `nh` huge blocks (`entries` in all) and completes
+// their words, units and tile counts -- unless some row's columns do not
+// ascend (cnt->odd), when nothing is completed.
+int merge_huge(const int *d_ptr, const int *d_idx, int rows, int nnz, int bm, int bn, int tilem, int cbits, int colA,
+               const Big *huge, unsigned nh, size_t entries, unsigned *words, Unit *units, int *nt, Counters *cnt,
+               hipStream_t s)
+{
+    Carve c;
+    const size_t k0 = c.add(8 * entries), k1 = c.add(8 * entries);
+    DevBufs db(s);
+    char *w = nullptr;
+    TCHK(db.get(&w, c.bytes));
+    unsigned long long *in = (unsigned long long *)(w + k0), *out = (unsigned long long *)(w + k1);
+    const dim3 grid(nh, kHugeY);
+    huge_keys_kernel<true><<<grid, kThreads, 0, s>>>(d_ptr, d_idx, rows, nnz, bm, tilem, cbits, colA, huge, in, nullptr,
+                                                     cnt);
+    for (int g = 1; g < bm; g *= 2) {
+        huge_merge_kernel<<<grid, kThreads, 0, s>>>(d_ptr, rows, nnz, bm, tilem, g, huge, in, out, cnt);
+        std::swap(in, out);
+    }
+    huge_words_kernel<true><<<grid, kThreads, 0, s>>>(d_ptr, rows, nnz, bm, tilem, huge, in, nullptr, words, units, cnt);
+    huge_ranks_kernel<<<nh, kThreads, 0, s>>>(d_ptr, rows, nnz, bm, bn, tilem, huge, units, nt, cnt, true);
+    return (int)hipGetLastError();
+}
+
+// The same by a radix sort, whatever the order of the rows' columns.
 int sort_huge(const int *d_ptr, const int *d_idx, int rows, int nnz, int bm, int bn, int tilem, int cbits, int colA,
               const Big *huge, unsigned nh, size_t entries, unsigned *words, Unit *units, int *nt, Counters *cnt,
               hipStream_t s)
@@ -976,13 +1269,13 @@ int sort_huge(const int *d_ptr, const int *d_idx, int rows, int nnz, int bm, int
     char *w = nullptr;
     TCHK(db.get(&w, c.bytes));
     const dim3 grid(nh, kHugeY);
-    huge_keys_kernel<<<grid, kThreads, 0, s>>>(d_ptr, d_idx, rows, nnz, bm, tilem, cbits, colA, huge,
-                                               (unsigned long long *)(w + k0), (unsigned *)(w + p0), cnt);
+    huge_keys_kernel<false><<<grid, kThreads, 0, s>>>(d_ptr, d_idx, rows, nnz, bm, tilem, cbits, colA, huge,
+                                                      (unsigned long long *)(w + k0), (unsigned *)(w + p0), cnt);
     TCHK(rocprim::radix_sort_pairs(w + t0, need, (unsigned long long *)(w + k0), (unsigned long long *)(w + k1),
                                    (unsigned *)(w + p0), (unsigned *)(w + p1), entries, 0, bits, s));
-    huge_words_kernel<<<grid, kThreads, 0, s>>>(d_ptr, rows, nnz, bm, tilem, huge, (unsigned long long *)(w + k1),
-                                                (unsigned *)(w + p1), words, units);
-    huge_ranks_kernel<<<nh, kThreads, 0, s>>>(d_ptr, rows, nnz, bm, bn, tilem, huge, units, nt);
+    huge_words_kernel<false><<<grid, kThreads, 0, s>>>(d_ptr, rows, nnz, bm, tilem, huge, (unsigned long long *)(w + k1),
+                                                       (unsigned *)(w + p1), words, units, cnt);
+    huge_ranks_kernel<<<nh, kThreads, 0, s>>>(d_ptr, rows, nnz, bm, bn, tilem, huge, units, nt, cnt, false);
     return (int)hipGetLastError();
 }
 
@@ -1022,7 +1315,7 @@ int tile_create_device(tsp_dev_tiles *out, int rows, int colA, long long nnz, co
     Carve cv;
     const size_t o_cnt = cv.add(sizeof(Counters)), o_state = cv.add(state_bytes);
     const size_t zeroed = cv.bytes;
-    const size_t o_nt = cv.add(4 * (size_t)tilem), o_medium = cv.add(sizeof(Big) * (size_t)medium_cap);
+    const size_t o_nt = cv.add(4 * (size_t)tilem), o_medium = cv.add(sizeof(Big) * 4 * (size_t)medium_cap);
     const size_t o_huge = cv.add(sizeof(Big) * (size_t)huge_cap), o_units = cv.add(sizeof(Unit) * (size_t)unit_cap);
     const size_t o_words = cv.add(4 * (size_t)n);
     DevBufs db(s);
@@ -1045,9 +1338,20 @@ int tile_create_device(tsp_dev_tiles *out, int rows, int colA, long long nnz, co
         sort_blocks_kernel<unsigned long long><<<wave_blocks, kThreads, 0, s>>>(
             d_ptr, d_idx, rows, n, BM, BN, tilem, cmask, colA, words, nt, medium, medium_cap, huge, huge_cap, unit_cap,
             cnt);
-    if (n > kSmall)
-        sort_medium_kernel<<<(unsigned)(medium_cap < 512 ? medium_cap : 512), kMediumThreads, 0, s>>>(
-            d_ptr, d_idx, rows, n, BM, BN, tilem, cmask, colA, words, nt, medium, medium_cap, units, cnt);
+    if (n > kSmall) {
+        // medium: two lists of blocks to merge, then room for both as blocks to sort
+        Big *unsorted = medium + 2 * (size_t)medium_cap;
+        const unsigned groups = (unsigned)(medium_cap < 2048 ? medium_cap : 2048);
+        merge_medium_kernel<kMedium / 2 / kMergePer><<<groups, kMedium / 2 / kMergePer, 0, s>>>(
+            d_ptr, d_idx, rows, n, BM, BN, tilem, cmask, colA, words, nt, medium, &cnt->nmerge[0], medium_cap, unsorted,
+            units, cnt);
+        if (n > kMedium / 2)
+            merge_medium_kernel<kMedium / kMergePer><<<groups, kMedium / kMergePer, 0, s>>>(
+                d_ptr, d_idx, rows, n, BM, BN, tilem, cmask, colA, words, nt, medium + medium_cap, &cnt->nmerge[1],
+                medium_cap, unsorted, units, cnt);
+        sort_medium_kernel<<<groups < 512 ? groups : 512, kMediumThreads, 0, s>>>(
+            d_ptr, d_idx, rows, n, BM, BN, tilem, cmask, words, nt, unsorted, 2 * medium_cap, units, cnt);
+    }
     TCHK(hipGetLastError());
     // 2. tile_ptr
     Counters h;
@@ -1057,9 +1361,10 @@ int tile_create_device(tsp_dev_tiles *out, int rows, int colA, long long nnz, co
         TCHK(hipStreamSynchronize(s));
         if (h.bad) return TSP_EINVAL;       // a column outside [0, colA)
         const size_t entries = (size_t)(h.huge & ((1ull << 40) - 1ull));
-        if (entries == 0 || pass) break;
-        if (int st = sort_huge(d_ptr, d_idx, rows, n, BM, BN, tilem, cbits, colA, huge, (unsigned)(h.huge >> 40), entries,
-                               words, units, nt, cnt, s))
+        if (entries == 0 || pass == 2 || (pass == 1 && !h.odd)) break;
+        const auto complete = pass ? sort_huge : merge_huge;
+        if (int st = complete(d_ptr, d_idx, rows, n, BM, BN, tilem, cbits, colA, huge, (unsigned)(h.huge >> 40), entries,
+                              words, units, nt, cnt, s))
             return st;
         TCHK(hipMemsetAsync(state, 0, state_bytes, s));
         TCHK(hipMemsetAsync(&cnt->ticket, 0, sizeof(int), s));
@@ -1097,7 +1402,7 @@ int tile_create_device(tsp_dev_tiles *out, int rows, int colA, long long nnz, co
             else fill(fill_kernel<float, 0, 0, DUP>, v);
         }
     };
-    if (h.dups) shape(std::true_type{});
+    if (h.dups || h.odd) shape(std::true_type{});
     else shape(std::false_type{});
     TCHK(hipGetLastError());
     return (int)hipStreamSynchronize(s);
