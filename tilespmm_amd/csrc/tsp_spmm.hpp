@@ -652,13 +652,22 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(k
                         }
                     }
                     __builtin_amdgcn_wave_barrier();
+                    // (reads in groups ahead of the tests, which would otherwise
+                    // each wait for its own)
+                    constexpr int NI = 8 * W / 64, GI = NI < 8 ? NI : 8;
 #pragma unroll
-                    for (int i = 0; i < 8 * W / 64; ++i) {
-                        const int idx = lane + 64 * i;
-                        const int rr = idx / W, col = idx % W;
-                        const int r = row0 + 8 * h + rr;
-                        const float x = tr[rr * W + col];
-                        if (r < c_rows && (!skip0 || x != 0.f)) unsafeAtomicAdd(C + (size_t)r * ld + col0 + col, x);
+                    for (int i0 = 0; i0 < NI; i0 += GI) {
+                        float x[GI];
+#pragma unroll
+                        for (int i = 0; i < GI; ++i) x[i] = tr[lane + 64 * (i0 + i)];
+#pragma unroll
+                        for (int i = 0; i < GI; ++i) {
+                            const int idx = lane + 64 * (i0 + i);
+                            const int rr = idx / W, col = idx % W;
+                            const int r = row0 + 8 * h + rr;
+                            // adding an exact zero changes nothing (NaN compares unequal)
+                            if (r < c_rows && x[i] != 0.f) unsafeAtomicAdd(C + (size_t)r * ld + col0 + col, x[i]);
+                        }
                     }
                     __builtin_amdgcn_wave_barrier();
                 }
