@@ -170,7 +170,8 @@ int tsp_spmm_launch_packed(int bm, int prec, int rowblkblock, int colB_p, const 
 
 /* Workgroup placement on the XCDs.  Each of the 8 XCDs of an MI355X has its
  * own L2 and receives every 8th workgroup of a launch.  The launches above
- * use TSP_PLACE_CONTIGUOUS: each XCD runs one contiguous eighth of the task
+ * use TSP_PLACE_CONTIGUOUS (16-row tiles at library defaults with 2, 4 or 8
+ * chunks: TSP_PLACE_CHUNK_XCD): each XCD runs one contiguous eighth of the task
  * ranges, so neighbouring row-blocks, which share B rows, share an L2.
  * TSP_PLACE_INTERLEAVED deals runs of 4 workgroups to the XCDs in turn,
  * which keeps matrices whose heavy rows sit together (graphs with hub

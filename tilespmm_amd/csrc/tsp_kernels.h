@@ -86,6 +86,9 @@ constexpr int kXcdRun = 4;
 constexpr int kPlaceContiguous = 0;
 constexpr int kPlaceInterleaved = 1;
 constexpr int kPlaceChunkXcd = 2;
+// The library chooses (launch()).
+constexpr int kPlaceAuto = -1;
+constexpr int kLaneAuto = -1;
 
 // Kernel option bits (the `opts` argument).
 constexpr int kOptSkipZeroStores = 1;   // do not store exact-zero results (C holds them already)
@@ -146,7 +149,7 @@ const void *select_kernel_bm8(int prec, int w, int s, bool packed, bool lane_idx
 int launch(int bm, int prec, int ntasks, int colB_p, const void *val, const uint64_t *bmp,
            const int *vptr, const unsigned *rows, const int *colstart, const void *B, float *C,
            const int *colidx, int c_rows, hipStream_t st, int w, int s, int tpw, int order,
-           int placement = kPlaceContiguous, bool lane_idx = false, int b_rows = 0, int panel_rows = 0,
+           int placement = kPlaceAuto, int lane = kLaneAuto, int b_rows = 0, int panel_rows = 0,
            int panel_lag = 1, int *sync = nullptr, long long sync_ints = 0, bool sync_reset = false,
            bool pair = false, int opts = 0);
 int launch_zero_rows(float *C, int c_rows, int colB_p, const int *units, int n, hipStream_t s);

@@ -144,16 +144,48 @@ constexpr int kSyncSpinUs = 20;
 int launch(int bm, int prec, int ntasks, int colB_p, const void *val, const uint64_t *bmp,
            const int *vptr, const unsigned *rows, const int *colstart, const void *B, float *C,
            const int *colidx, int c_rows, hipStream_t st, int w, int s, int tpw, int order,
-           int placement, bool lane_idx, int b_rows, int panel_rows, int panel_lag, int *sync, long long sync_ints,
+           int placement, int lane, int b_rows, int panel_rows, int panel_lag, int *sync, long long sync_ints,
            bool sync_reset, bool pair, int opts)
 {
     const bool packed = bmp != nullptr;
     if (packed && (bm == 64 || !vptr)) return TSP_EINVAL;
     const bool library_tpw = tpw <= 0;
+    const bool auto_w = w <= 0, auto_s = s <= 0, auto_all = auto_w && auto_s && tpw <= 0 && order <= 0;
+    const bool auto_place = placement == kPlaceAuto && auto_all, auto_lane = lane == kLaneAuto && auto_all;
+    if (placement == kPlaceAuto) placement = kPlaceContiguous;
     if (placement != kPlaceContiguous && placement != kPlaceInterleaved && placement != kPlaceChunkXcd)
         return TSP_EINVAL;
     int nchunks = 0, cm = 0;
     if (!resolve_variant(bm, prec, colB_p, w, s, nchunks, tpw, order, cm)) return TSP_EINVAL;
+    const bool plain = !sync && !pair;
+    // What a launch leaves to the library, from launches of every class,
+    // format and precision at 12 matrices each:
+    //   * fewer than 12 waves per CU: narrower chunks, which make more waves
+    //     (banded 3000 tf32 n=256, 16-row: 17.6 -> 11.7 us at 32 columns
+    //     instead of 128, 8-row 1.20x; from 3750 waves on 16-row tiles lose
+    //     by it, block-sparse 0.86x); 64-row fp16 tiles are left alone (0.8x
+    //     to 1.18x);
+    const long long few = bm == 64 ? (prec == TSP_PREC_FP16 ? 0 : 4096) : 3072;
+    if (plain && auto_w && placement != kPlaceChunkXcd)
+        while (w > 32 && (long long)ntasks * nchunks < few) {
+            w /= 2;
+            nchunks = colB_p / w;
+        }
+    const long long waves1 = (long long)ntasks * nchunks;    // of one task each
+    //   * 64-row tf32 tiles (64 fp32 MFMAs a tile): two tiles in flight where
+    //     few waves hide each other's latency (1.07x);
+    if (plain && auto_s && bm == 64 && prec != TSP_PREC_FP16 && waves1 < 4096) s = 2;
+    //   * 16-row tiles with 2, 4 or 8 chunks: one chunk per group of XCDs,
+    //     whose L2s then share out B's columns (1.04x over 24 launches, 0.96x
+    //     at worst; block-sparse 65536 fp16 n=256 349 -> 293 us);
+    if (plain && auto_place && bm == 16 && (nchunks == 2 || nchunks == 4 || nchunks == 8))
+        placement = kPlaceChunkXcd;
+    //   * column indices loaded per lane for small launches, which wait for
+    //     the select chain (1.05x, 0.94x at worst), and for tf32 8-row tiles
+    //     (1.03x); fp16 8-row tiles of large launches lose (0.79x).
+    bool lane_idx = lane == 1;
+    if (auto_lane)
+        lane_idx = plain && bm <= 16 && (packed || w <= 128) && (waves1 <= 4096 || (bm == 8 && prec != TSP_PREC_FP16));
     if (placement == kPlaceChunkXcd && (nchunks < 2 || kXcds % nchunks != 0)) return TSP_EINVAL;
     // Sums of split row-blocks added up in the workgroup, where the tasks per
     // wave are the library's: four tasks of a chunk to a workgroup, or two of
