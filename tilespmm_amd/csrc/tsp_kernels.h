@@ -126,19 +126,15 @@ int default_chunk_width(int bm, int colB_p);
 int default_stages(int bm, int prec, int w);
 bool valid_variant(int bm, int w, int s);
 const void *select_kernel(int bm, int prec, int w, int s, bool packed, bool lane_idx = false, bool sync = false,
-                          bool pair = false, bool sum = false);
+                          bool pair = false);
 // The instantiations of one row-block class (tsp_spmm_bm{64,16,8}.hip);
 // nullptr for a variant that is not built.  prec: TSP_PREC_FP16,
 // TSP_PREC_TF32, kPrecTf32Exact or kPrecTf32B3.  pair: the tile-pair form
 // (fp16 8- and 16-row tiles at 64- and 128-column chunks; kPrecTf32Exact
-// 8-row tiles at 64-column chunks).  sum: split row-blocks' sums added up in
-// the workgroup (depth 1, chunks of up to 128 columns, no pairs, no sweep).
-const void *select_kernel_bm64(int prec, int w, int s, bool packed, bool lane_idx, bool sync, bool pair,
-                               bool sum);
-const void *select_kernel_bm16(int prec, int w, int s, bool packed, bool lane_idx, bool sync, bool pair,
-                               bool sum);
-const void *select_kernel_bm8(int prec, int w, int s, bool packed, bool lane_idx, bool sync, bool pair,
-                               bool sum);
+// 8-row tiles at 64-column chunks).
+const void *select_kernel_bm64(int prec, int w, int s, bool packed, bool lane_idx, bool sync, bool pair);
+const void *select_kernel_bm16(int prec, int w, int s, bool packed, bool lane_idx, bool sync, bool pair);
+const void *select_kernel_bm8(int prec, int w, int s, bool packed, bool lane_idx, bool sync, bool pair);
 // w, s, tpw <= 0 select the defaults; order 0 = default, 1 = chunks of one
 // task range adjacent, 2 = chunk-major.  bmp != nullptr selects the
 // bitmap-packed A format (val = packed values, vptr = per-tile offsets).

@@ -88,11 +88,11 @@ bool valid_variant(int bm, int w, int s)
     return w == 32 || w == 64 || w == 128;
 }
 
-const void *select_kernel(int bm, int prec, int w, int s, bool packed, bool lane_idx, bool sync, bool pair, bool sum)
+const void *select_kernel(int bm, int prec, int w, int s, bool packed, bool lane_idx, bool sync, bool pair)
 {
-    if (bm == 64) return select_kernel_bm64(prec, w, s, packed, lane_idx, sync, pair, sum);
-    if (bm == 16) return select_kernel_bm16(prec, w, s, packed, lane_idx, sync, pair, sum);
-    if (bm == 8) return select_kernel_bm8(prec, w, s, packed, lane_idx, sync, pair, sum);
+    if (bm == 64) return select_kernel_bm64(prec, w, s, packed, lane_idx, sync, pair);
+    if (bm == 16) return select_kernel_bm16(prec, w, s, packed, lane_idx, sync, pair);
+    if (bm == 8) return select_kernel_bm8(prec, w, s, packed, lane_idx, sync, pair);
     return nullptr;
 }
 
@@ -149,7 +149,6 @@ int launch(int bm, int prec, int ntasks, int colB_p, const void *val, const uint
 {
     const bool packed = bmp != nullptr;
     if (packed && (bm == 64 || !vptr)) return TSP_EINVAL;
-    const bool library_tpw = tpw <= 0;
     const bool auto_w = w <= 0, auto_s = s <= 0, auto_all = auto_w && auto_s && tpw <= 0 && order <= 0;
     const bool auto_place = placement == kPlaceAuto && auto_all, auto_lane = lane == kLaneAuto && auto_all;
     if (placement == kPlaceAuto) placement = kPlaceContiguous;
@@ -177,7 +176,7 @@ int launch(int bm, int prec, int ntasks, int colB_p, const void *val, const uint
     if (plain && auto_s && bm == 64 && prec != TSP_PREC_FP16 && waves1 < 4096) s = 2;
     //   * 16-row tiles with 2, 4 or 8 chunks: one chunk per group of XCDs,
     //     whose L2s then share out B's columns (1.04x over 24 launches, 0.96x
-    //     at worst; block-sparse 65536 fp16 n=256 349 -> 293 us);
+    //     at worst; block-sparse 65536 fp16 n=256 337 -> 267 us);
     if (plain && auto_place && bm == 16 && (nchunks == 2 || nchunks == 4 || nchunks == 8))
         placement = kPlaceChunkXcd;
     //   * column indices loaded per lane for small launches, which wait for
@@ -187,22 +186,11 @@ int launch(int bm, int prec, int ntasks, int colB_p, const void *val, const uint
     if (auto_lane)
         lane_idx = plain && bm <= 16 && (packed || w <= 128) && (waves1 <= 4096 || (bm == 8 && prec != TSP_PREC_FP16));
     if (placement == kPlaceChunkXcd && (nchunks < 2 || kXcds % nchunks != 0)) return TSP_EINVAL;
-    // Sums of split row-blocks added up in the workgroup, where the tasks per
-    // wave are the library's: four tasks of a chunk to a workgroup, or two of
-    // two chunks (one chunk's waves beside each other read A once: four tasks
-    // of one of several chunks ran a Laplacian 25% slower).
-    const bool whole = nchunks == 1 || cm || placement == kPlaceChunkXcd;
-    // 64-row tiles meet at 15 barriers, which small launches feel (uniform
-    // 8000 x 8000 fp16, 250 tasks: 13.2 -> 15.9 us; power law 300000, 40000
-    // tasks: 1.9x faster).
-    const bool sum = library_tpw && !sync && !pair && s == 1 && w <= 128 && (whole || nchunks % 2 == 0) &&
-                     (bm < 64 || (long long)ntasks * nchunks >= 4096);
-    const void *k = select_kernel(bm, prec, w, s, packed, lane_idx, sync != nullptr, pair, sum);
+    const void *k = select_kernel(bm, prec, w, s, packed, lane_idx, sync != nullptr, pair);
     if (!k) return TSP_EINVAL;
     const long long ranges = ((long long)ntasks + tpw - 1) / tpw;
     const long long waves = ranges * nchunks;
     long long blocks = (waves + kWavesPerBlock - 1) / kWavesPerBlock;
-    if (sum) blocks = whole ? (ranges + kWavesPerBlock - 1) / kWavesPerBlock * nchunks : (ranges + 1) / 2 * (nchunks / 2);
     if (blocks <= 0) return 0;
     SyncArgs sy{nullptr, 0, 1, 0, 1, 1, 0};
     if (sync) {

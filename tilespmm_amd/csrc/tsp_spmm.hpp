@@ -123,14 +123,8 @@ __device__ __forceinline__ u4 widen_3byte(u4 p)
 // in 72): their widening's temporaries cost up to 6 registers more.  (The
 // LDS-panel ones widen before the LDS write and need fewer registers than
 // their 4-byte counterparts.)
-// The forms that add up sums in the workgroup (CO) are held to the waves of
-// their plain counterparts where they land one or two registers past them.
-template <int BM, int W, int PREC, int S, bool PK, bool LI, bool SY, bool PR, bool CO>
-constexpr int kMinWaves = CO && PK && ((BM == 8 && W == 64 && PREC == TSP_PREC_FP16 && !LI) ||
-                                       (BM == 16 && W == 64 && (PREC == TSP_PREC_FP16 || PREC == kPrecTf32Exact) && LI)) ? 8
-                          : CO && W == 128 && PREC == kPrecTf32B3 && !LI && PK == (BM == 8) && BM <= 16 ? 6
-                          : CO && W == 128 && PREC == TSP_PREC_FP16 && !LI && PK && BM == 8             ? 5
-                          : PR ? (SY && W == 64 && S == 1 ? 5 : 1)
+template <int BM, int W, int PREC, int S, bool PK, bool SY, bool PR>
+constexpr int kMinWaves = PR ? (SY && W == 64 && S == 1 ? 5 : 1)
                           : PREC == kPrecTf32B3 && BM <= 16 && W == 64 ? (S == 3 ? 5 : S == 2 && BM == 8 ? 7 : 1)
                           : BM == 64 && W == 64 && S == 1 && !SY                                      ? 3
                           : SY && PREC == TSP_PREC_FP16 && BM == 16 && W == 128 && S == 1 ? 5
@@ -149,17 +143,8 @@ constexpr int kMinWaves = CO && PK && ((BM == 8 && W == 64 && PREC == TSP_PREC_F
 // split-bf16 products on v_mfma_f32_16x16x32_bf16 (SPL below).  A task with
 // an odd number of tiles ends with a unit whose second half has zero A
 // values and zeroed B rows.
-// CO: sums of split row-blocks added up in the workgroup.  One task per wave;
-// the workgroup holds four consecutive tasks of one chunk, or two of two
-// neighbouring chunks, and the waves whose tasks are of one split row-block
-// put their sums side by side in LDS and add them to C once.  C's atomics
-// bound the launches of skewed matrices (RMAT scale 18, fp16 16-row tiles, 64
-// columns: 206 us, 80 us without any); with this 90 us, RMAT scale 20 fp16
-// 8-row packed at 128 columns 1.41 -> 1.08 ms, a circuit of 117k rows at 32
-// columns 20 -> 15 us.  Merging the tasks on one wave instead saves as many
-// atomics but idles the others: 0.93x over 120 launches, against 1.12x.
-template <int BM, int W, int PREC, int S, bool PK, bool LI, bool SY, bool PR = false, bool CO = false>
-__global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(kMinWaves<BM, W, PREC, S, PK, LI, SY, PR, CO>))) void spmm_kernel(
+template <int BM, int W, int PREC, int S, bool PK, bool LI, bool SY, bool PR = false>
+__global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(kMinWaves<BM, W, PREC, S, PK, SY, PR>))) void spmm_kernel(
     int ntasks, int nchunks, int tasks_per_wave, int chunk_major, const void *__restrict__ val_,
     const uint64_t *__restrict__ bmp, const int *__restrict__ vptr,
     const unsigned *__restrict__ rows, const int *__restrict__ colstart,
@@ -247,7 +232,7 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(k
     // skip the 64-bit divisions: each costs dozens of scalar instructions,
     // which a launch-bound kernel pays in full)
     const long long nranges =
-        CO || tasks_per_wave == 1 ? (long long)ntasks : ((long long)ntasks + tasks_per_wave - 1) / tasks_per_wave;
+        tasks_per_wave == 1 ? (long long)ntasks : ((long long)ntasks + tasks_per_wave - 1) / tasks_per_wave;
     const bool sync = SY && sy.cnt != nullptr;
     const int xcd = blockIdx.x % kXcds;
     // Counters of generation g on this XCD: the waves registered for it, then
@@ -279,38 +264,16 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(k
             for (int i = from; i <= to; ++i) bump(g, 1 + i);
     };
 
-    // CO: whether the workgroup holds two tasks of two chunks; the waves whose
-    // tasks are of this wave's split row-block.
-    static_assert(!CO || (!SY && !PR), "sums in the workgroup: one task per wave, single tiles, no panel sweep");
-    const bool two_chunks = CO && nchunks > 1 && !chunk_major && placement != kPlaceChunkXcd;
-    unsigned peers = 0;
-    auto find_peers = [&](int k, unsigned rw) {
-        const int step = two_chunks ? 2 : 1, first = two_chunks ? wid & 1 : 0, base = k - wid / step;
-#pragma unroll
-        for (int i = 0; i < kWavesPerBlock; ++i) {
-            const int ki = min(base + i, ntasks - 1);
-            const bool same = base + i < ntasks && uload(rows, ki) == rw && uload(colstart, ki + 1) > uload(colstart, ki);
-            if (first + i * step < kWavesPerBlock) peers |= same ? 1u << (first + i * step) : 0u;
-        }
-    };
-    // Only waves with peers stop at barriers, 2 (BM / 8) - 1 times each; a
-    // barrier waits for the workgroup's waves that have not ended.
-    auto barrier = [&]() {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-    };
-
     // One work item: the task range `range` on column chunk `chunk`.
     auto run = [&](int g, int range, int chunk) {
         int lp = -1;                     // last panel this wave announced (sync)
-        const int k0 = CO ? range : range * tasks_per_wave;
-        const int k1 = CO ? k0 + 1 : min(ntasks, k0 + tasks_per_wave);
+        const int k0 = range * tasks_per_wave;
+        const int k1 = min(ntasks, k0 + tasks_per_wave);
         // One batch of scalar loads: the range's tile bounds, the first task's
         // end and its schedule word (first row, split flag; a task's word is
         // read when the task starts, so that a flush never waits for it).
         const int tb = uload(colstart, k0), te = uload(colstart, k1);
-        int kend = CO ? te : uload(colstart, k0 + 1);
+        int kend = uload(colstart, k0 + 1);
         unsigned rwk = uload(rows, k0);
         if (tb >= te) return;                        // every task of the range is empty
         // a wave waits only for the waves that registered before it looks, so
@@ -322,7 +285,7 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(k
         // are in flight, so that the common case (none) adds no round trip
         // before them.
         auto skip_empty = [&]() {
-            if (CO || kend > tb) return;
+            if (kend > tb) return;
             while (kend <= tb) kend = uload(colstart, ++k + 1);
             gfirst = k;
             rwk = uload(rows, k);
@@ -612,8 +575,7 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(k
         // and is stored (the test per stored value or vector cost nothing
         // measurable on configurations 2 and 4, which have no empty rows).
         const bool skip0 = (opts & kOptSkipZeroStores) != 0;
-        // tf32 tile pairs: the row sums of the two halves of A
-        auto fold_halves = [&]() {
+        auto flush = [&](int first, int last, unsigned rw) {   // rw = rows[last]
             if constexpr (SPL) {
                 // rows 8-15 of each MFMA block hold the low-half products of
                 // rows 0-7: lane l (< 32) adds lane l + 32's sums.  Where an
@@ -629,32 +591,6 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(k
                         acc[0][c][j] = __builtin_isinf(acc[0][c][j]) ? acc[0][c][j] : acc[0][c][j] + o;
                     }
             }
-        };
-        // One 8-row slab of the accumulators into the wave's (now idle) B
-        // panel in LDS, rows of W consecutive columns: fp32 atomics are issued
-        // per lane, and this way every atomic instruction covers whole rows.
-        static_assert(BNU * LDSW * sizeof(VT) >= 8 * W * sizeof(float), "panel too small for a slab");
-        auto put_slab = [&](int h) {
-            float *tr = (float *)lds;
-            if ((lq >> 1) == (h & 1)) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    float *trow = tr + (4 * (lq & 1) + j) * W;
-                    if constexpr (TR) {
-#pragma unroll
-                        for (int c = 0; c < CB; ++c) trow[16 * c + ln] = acc[h >> 1][c][j];
-                    } else {
-                        FV v;
-#pragma unroll
-                        for (int c = 0; c < CB; ++c) v[c] = acc[h >> 1][c][j];
-                        *(FV *)(trow + ln * CB) = v;
-                    }
-                }
-            }
-        };
-        constexpr int NI = 8 * W / 64, GI = NI < 8 ? NI : 8;   // reads of a slab, and how many at once
-        auto flush = [&](int first, int last, unsigned rw) {   // rw = rows[last]
-            fold_halves();
             const int row0 = (int)(rw & 0x7fffffffu);
             bool split = (rw & 0x80000000u) != 0;
             if (split && first < last) {
@@ -693,13 +629,32 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(k
                     }
                 }
             } else {
-                const float *tr = (const float *)lds;
+                // fp32 atomics are issued per lane: transpose each 8-row slab
+                // through the wave's (now idle) B panel in LDS so that every
+                // atomic instruction covers whole rows of consecutive columns
+                static_assert(BNU * LDSW * sizeof(VT) >= 8 * W * sizeof(float), "panel too small for a slab");
+                float *tr = (float *)lds;
 #pragma unroll
                 for (int h = 0; h < BM / 8; ++h) {
-                    put_slab(h);
+                    if ((lq >> 1) == (h & 1)) {
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            float *trow = tr + (4 * (lq & 1) + j) * W;
+                            if constexpr (TR) {
+#pragma unroll
+                                for (int c = 0; c < CB; ++c) trow[16 * c + ln] = acc[h >> 1][c][j];
+                            } else {
+                                FV v;
+#pragma unroll
+                                for (int c = 0; c < CB; ++c) v[c] = acc[h >> 1][c][j];
+                                *(FV *)(trow + ln * CB) = v;
+                            }
+                        }
+                    }
                     __builtin_amdgcn_wave_barrier();
                     // (reads in groups ahead of the tests, which would otherwise
                     // each wait for its own)
+                    constexpr int NI = 8 * W / 64, GI = NI < 8 ? NI : 8;
 #pragma unroll
                     for (int i0 = 0; i0 < NI; i0 += GI) {
                         float x[GI];
@@ -721,37 +676,6 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(k
             for (int g = 0; g < RG; ++g)
 #pragma unroll
                 for (int c = 0; c < CB; ++c) acc[g][c] = f4{0.f, 0.f, 0.f, 0.f};
-        };
-        // The end of the wave's tasks.  Where several waves of the workgroup
-        // hold sums of one split row-block, they put them side by side in LDS,
-        // slab by slab, and share out the adding up and the atomics.
-        auto finish = [&](int first, int last, unsigned rw) {
-            // (looked up here, not ahead of the first loads, which would wait
-            // for the schedule word)
-            if constexpr (CO) {
-                if (rw & 0x80000000u) find_peers(last, rw);
-            }
-            if (!CO || (peers & (peers - 1)) == 0) {
-                flush(first, last, rw);
-                return;
-            }
-            const int row0 = (int)(rw & 0x7fffffffu);
-            const int np = __popc(peers), me = __popc(peers & ((1u << wid) - 1u));
-#pragma unroll
-            for (int h = 0; h < BM / 8; ++h) {
-                put_slab(h);
-                barrier();
-                for (int i = me; i < NI; i += np) {
-                    const int idx = lane + 64 * i;
-                    float x = 0.f;
-#pragma unroll
-                    for (int w = 0; w < kWavesPerBlock; ++w)
-                        if (peers >> w & 1u) x += ((const float *)lds_all[w])[idx];
-                    const int r = row0 + 8 * h + idx / W;
-                    if (r < c_rows && x != 0.f) unsafeAtomicAdd(C + (size_t)r * ld + col0 + idx % W, x);
-                }
-                if (h + 1 < BM / 8) barrier();
-            }
         };
         // B operand of MFMA block c at lane (n = ln, group lq).  Dense fp16
         // (TR): column 16c + n of the chunk, read with LDS transpose reads
@@ -919,7 +843,7 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(k
         // Task bookkeeping when the compute front reaches tile t: at the end
         // of task k, flush unless the next task continues the same row-block.
         auto advance_task = [&](int t) {
-            if (!CO && t >= kend) {                 // task k is complete
+            if (t >= kend) {                 // task k is complete
                 int kn = k;
                 do kend = uload(colstart, ++kn + 1);
                 while (kend <= t);           // skip empty tasks
@@ -1020,7 +944,7 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(k
                     }
                 }
             }
-            finish(gfirst, k, rwk);
+            flush(gfirst, k, rwk);
             if (sync && lp < sy.npanels - 1) announce(g, lp + 1, sy.npanels - 1);
             return;
         }
@@ -1072,7 +996,7 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(k
                 }
             }
         }
-        finish(gfirst, k, rwk);
+        flush(gfirst, k, rwk);
         if (sync && lp < sy.npanels - 1) announce(g, lp + 1, sy.npanels - 1);
     };
 
@@ -1092,21 +1016,6 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(k
                 r = rr;
                 chunk = x % nchunks;
             }
-        } else if constexpr (CO) {
-            const int lb = place_block(blockIdx.x, gridDim.x, placement);
-            int k = lb * kWavesPerBlock + wid;
-            if (two_chunks) {
-                const unsigned half = (unsigned)nchunks / 2;
-                const int t2 = (half & (half - 1)) == 0 ? lb >> __builtin_ctz(half) : lb / (int)half;
-                chunk = 2 * (lb - t2 * (int)half) + (wid & 1);
-                k = 2 * t2 + wid / 2;
-            } else if (nchunks > 1) {
-                const int groups = (ntasks - 1) / kWavesPerBlock + 1;
-                int l = lb;
-                for (; l >= groups; l -= groups) ++chunk;
-                k = l * kWavesPerBlock + wid;
-            }
-            if (k < ntasks && chunk < nchunks) r = k;
         } else {
             const int lb = place_block(blockIdx.x, gridDim.x, placement);
             const long long gw = ((long long)g * gridDim.x + lb) * kWavesPerBlock + wid;
@@ -1115,20 +1024,11 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(k
                 // (the live B working set of a phase is one chunk's columns);
                 // otherwise the chunks of one range are neighbours (the A
                 // tiles are reused from L2).
-                // (no 64-bit division where it can be helped: it costs a
-                // wave over a hundred scalar instructions before its first
-                // load)
                 if (nchunks == 1) {
                     r = gw;
-                } else if (chunk_major) {
-                    r = gw;
-                    for (; r >= nranges; r -= nranges) ++chunk;
-                } else if ((nchunks & (nchunks - 1)) == 0) {
-                    r = gw >> __builtin_ctz((unsigned)nchunks);
-                    chunk = (int)gw & (nchunks - 1);
                 } else {
-                    r = gw / nchunks;
-                    chunk = (int)(gw - r * nchunks);
+                    r = chunk_major ? gw % nranges : gw / nchunks;
+                    chunk = chunk_major ? (int)(gw / nranges) : (int)(gw - r * nchunks);
                 }
             }
         }
@@ -1139,16 +1039,16 @@ __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(k
 // Host-side address of one instantiation for a launch precision
 // (TSP_PREC_FP16, TSP_PREC_TF32, kPrecTf32Exact, or kPrecTf32B3 without the
 // panel sweep -- nullptr with it); taking it instantiates the kernel.
-template <int BM, int W, int S, bool PK, bool LI, bool SY, bool CO = false>
+template <int BM, int W, int S, bool PK, bool LI, bool SY>
 const void *pick_kernel(int prec)
 {
-    if (prec == TSP_PREC_FP16) return (const void *)&spmm_kernel<BM, W, TSP_PREC_FP16, S, PK, LI, SY, false, CO>;
-    if (prec == kPrecTf32Exact) return (const void *)&spmm_kernel<BM, W, kPrecTf32Exact, S, PK, LI, SY, false, CO>;
+    if (prec == TSP_PREC_FP16) return (const void *)&spmm_kernel<BM, W, TSP_PREC_FP16, S, PK, LI, SY>;
+    if (prec == kPrecTf32Exact) return (const void *)&spmm_kernel<BM, W, kPrecTf32Exact, S, PK, LI, SY>;
     if (prec == kPrecTf32B3) {
-        if constexpr (!SY) return (const void *)&spmm_kernel<BM, W, kPrecTf32B3, S, PK, LI, SY, false, CO>;
+        if constexpr (!SY) return (const void *)&spmm_kernel<BM, W, kPrecTf32B3, S, PK, LI, SY>;
         return nullptr;
     }
-    return (const void *)&spmm_kernel<BM, W, TSP_PREC_TF32, S, PK, LI, SY, false, CO>;
+    return (const void *)&spmm_kernel<BM, W, TSP_PREC_TF32, S, PK, LI, SY>;
 }
 
 // Tile-pair instantiations: fp16, and tf32 operands that are tf32 values

@@ -7,21 +7,8 @@
 
 namespace tsp {
 
-const void *select_kernel_bm16(int prec, int w, int s, bool packed, bool lane_idx, bool sync, bool pair,
-                               bool sum)
+const void *select_kernel_bm16(int prec, int w, int s, bool packed, bool lane_idx, bool sync, bool pair)
 {
-    if (sum) {
-        // depth 1, chunks of up to 128 columns
-        if (s != 1 || sync || pair) return nullptr;
-#define TSP_S(Wv, PKv, LIv)                                \
-    if (w == Wv && packed == PKv && lane_idx == LIv) \
-        return pick_kernel<16, Wv, 1, PKv, LIv, false, true>(prec);
-#define X(Wv) TSP_S(Wv, false, false) TSP_S(Wv, false, true) TSP_S(Wv, true, false) TSP_S(Wv, true, true)
-        X(32) X(64) X(128)
-#undef X
-#undef TSP_S
-        return nullptr;
-    }
     if (pair) {
         // tile pairs (fp16): 64- and 128-column chunks
 #define TSP_P(Wv, Sv, PKv, LIv, SYv)                                                  \

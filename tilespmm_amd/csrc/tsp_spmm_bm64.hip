@@ -5,19 +5,8 @@
 
 namespace tsp {
 
-const void *select_kernel_bm64(int prec, int w, int s, bool packed, bool lane_idx, bool sync, bool pair,
-                               bool sum)
+const void *select_kernel_bm64(int prec, int w, int s, bool packed, bool lane_idx, bool sync, bool pair)
 {
-    if (sum) {
-        // depth 1, chunks of up to 64 columns
-        if (s != 1 || sync || pair) return nullptr;
-#define TSP_S(Wv, PKv, LIv)                                \
-    if (w == Wv && packed == PKv && lane_idx == LIv) \
-        return pick_kernel<64, Wv, 1, PKv, LIv, false, true>(prec);
-        TSP_S(32, false, false) TSP_S(64, false, false)
-#undef TSP_S
-        return nullptr;
-    }
     if (pair) return nullptr;   // 64-row fp16 tiles are 32 wide already (K = 32)
 #define TSP_K(Wv, Sv, PKv, LIv, SYv)                                                  \
     if (w == Wv && s == Sv && packed == PKv && lane_idx == LIv && sync == SYv) \

@@ -34,7 +34,6 @@ struct ClassDev {
     long long cap_tasks = 0;
     int th = 0;
     int ntasks = 0;
-    bool any_split = false;       // the schedule has split tasks
     int var_w = 0, var_s = 0, var_tpw = 0, var_order = 0;   // kernel variant, 0 = library default
     int var_li = 0;               // lane-loaded column indices (TSP_LAUNCH_LANE_INDICES), where a kernel has them
     int wdef = 0;                 // the library's default chunk width for this class
@@ -149,8 +148,6 @@ static int upload_schedule(tsp_plan *p, ClassDev &c, int th)
     TSP_TRY(tsp_memcpy_h2d(c.d_colstart, it->second.second.data(), sizeof(int) * ((size_t)n + 1)));
     c.th = th;
     c.ntasks = n;
-    c.any_split = false;
-    for (unsigned r : it->second.first) c.any_split |= (r & 0x80000000u) != 0;
     p->zero_fresh = false;
     // Mirror the schedule into the tile matrix, as update_metadata does.
     free(c.m->blkcoostylerowidx);
@@ -270,10 +267,6 @@ static int launch_class(tsp_plan *p, ClassDev &c, void *stream = nullptr)
     if (!c.active() || c.ntasks == 0) return TSP_OK;
     const bool pk = c.fmt == 2;
     const bool b3 = b3_on(p, c);
-    // The library's default adds up split row-blocks in the workgroup; without
-    // any, the plain kernel is the better one (5-point Laplacian 512^2 fp16
-    // n=128: 35.0 us against 36.8).
-    const int tpw = c.var_tpw > 0 || c.any_split ? c.var_tpw : 1;
     const int flags = (p->prec == TSP_PREC_TF32 ? TSP_LAUNCH_OPERANDS_TF32 : 0) |
                       (lane_indices_on(c) ? TSP_LAUNCH_LANE_INDICES : 0) | (c.var_pr ? TSP_LAUNCH_TILE_PAIRS : 0) |
                       (p->c_shared ? 0 : TSP_LAUNCH_SKIP_ZERO_STORES) | (b3 ? TSP_LAUNCH_B_3BYTE : 0);
@@ -295,7 +288,7 @@ static int launch_class(tsp_plan *p, ClassDev &c, void *stream = nullptr)
                               pk ? c.d_vptr : nullptr, c.d_rows, c.d_colstart,
                               reads_split_b(p, c) ? p->d_Bs : b3 ? p->d_B3 : p->d_B,
                               p->d_C, c.d_colidx, p->rowA,
-                              stream ? stream : c.stream, c.var_w, c.var_s, tpw, c.var_order, c.place, flags);
+                              stream ? stream : c.stream, c.var_w, c.var_s, c.var_tpw, c.var_order, c.place, flags);
 }
 
 extern "C" int tsp_plan_set_panels(tsp_plan *p, int bm, int panel_rows, int lag)
